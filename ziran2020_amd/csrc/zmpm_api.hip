@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -13,6 +14,7 @@
 #include <limits>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 using namespace zmpm;
@@ -123,6 +125,15 @@ struct zmpm_context {
         hipGraphExec_t exec;
     };
     std::vector<Graph> graphs;
+    // pinned download buffers, one per participating host thread, and the word
+    // in which a download reports a corrupt id table
+    struct Slot {
+        void* host = nullptr;
+        size_t size = 0;
+        hipEvent_t done = nullptr;
+    };
+    std::vector<Slot> dl_slots;
+    int* dl_bad = nullptr;
     bool use_graphs = true;
     int fj_state = 0;       // FJMixedMpmForceHelper::state: 0 SOLVE_F, 1 SOLVE_J
     hipError_t launch_err = hipSuccess; // a failed launch that returns its error (the cooperative k_cg)
@@ -266,6 +277,7 @@ zmpm_status allocate(zmpm_context* h, int n)
     ALLOC(D.perm, cap);
     ALLOC(D.sorted_cell, cap);
     ALLOC(D.spid, cap);
+    ALLOC(D.inv, cap);
     ALLOC(D.touched, D.num_pages);
     ALLOC(D.page_count, D.num_pages);
     ALLOC(D.page_table, D.num_pages);
@@ -329,6 +341,7 @@ zmpm_status allocate(zmpm_context* h, int n)
     HIPCHK(h, hipMemsetAsync(D.perm, 0, cap * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.sorted_cell, 0, cap * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.spid, 0, cap * sizeof(int), h->stream));
+    HIPCHK(h, hipMemsetAsync(D.inv, 0, cap * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.counters, 0, 8 * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.maxbits, 0, ns * NSC * BOUND_SLOTS * sizeof(unsigned int), h->stream));
     const std::vector<float> ones((size_t)(NSC * ns), 1.f);
@@ -677,12 +690,6 @@ int encodePos(double x, double dx, int pb)
     return (int)u;
 }
 
-double decodePos(int X, double dx, int pb)
-{
-    if (X == POS_NAN) return std::numeric_limits<double>::quiet_NaN();
-    return (double)X * dx / (double)(1 << pb);
-}
-
 template <class T, class AccT>
 zmpm_status uploadT(zmpm_context* h, const zmpm_particles* p, const int32_t* scene)
 {
@@ -784,52 +791,118 @@ zmpm_status restress(zmpm_context* h)
     return ZMPM_OK;
 }
 
+// Downloads go through pinned buffers of at most kSlotBytes, one per
+// participating host thread: each thread takes the next range of words, has
+// k_export write it into its buffer and copies it on to the caller's arrays, so
+// the transfer of one range runs beside the host copies of the others.
+constexpr size_t kSlotBytes = 4u << 20;
+constexpr int kMaxSlots = 8;
+
+// The handle's pinned buffers for `want` participants and `bytes` in all (kept
+// until the handle ends, 32 MiB at most; a buffer grows to what is asked of it).
+zmpm_status downloadSlots(zmpm_context* h, int want, size_t bytes)
+{
+    if (!h->dl_bad) HIPCHK(h, hipHostMalloc((void**)&h->dl_bad, sizeof(int)));
+    while ((int)h->dl_slots.size() < want) {
+        zmpm_context::Slot sl;
+        HIPCHK(h, hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
+        h->dl_slots.push_back(sl);
+    }
+    for (int k = 0; k < want; k++) {
+        zmpm_context::Slot& sl = h->dl_slots[(size_t)k];
+        const size_t need = std::min(kSlotBytes, std::max<size_t>(bytes, 4096));
+        if (sl.size >= need) continue;
+        if (sl.host) (void)hipHostFree(sl.host);
+        sl.host = nullptr;
+        sl.size = 0;
+        if (hipHostMalloc(&sl.host, need) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(h, ZMPM_E_NOMEM, "no pinned memory for the download");
+        }
+        sl.size = need;
+    }
+    return ZMPM_OK;
+}
+
 template <class T, class AccT>
 zmpm_status downloadT(zmpm_context* h, zmpm_particles* p)
 {
-    Dev<T, AccT>& D = devOf<T, AccT>(h);
-    const int n = h->n;
-    const int64_t cap = D.cap;
-    std::vector<T> buf((size_t)NPF * cap);
-    std::vector<int> ids(cap), mat(cap);
-    HIPCHK(h, hipMemcpyAsync(buf.data(), D.P, buf.size() * sizeof(T), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(ids.data(), D.pid, cap * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipMemcpyAsync(mat.data(), D.pmat, cap * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int s = 0; s < n; s++) {
-        const int i = ids[s];
-        if (i < 0 || i >= n) return fail(h, ZMPM_E_HIP, "corrupt particle id table");
-        const int sc = mat[s] >> PMAT_SCENE_SHIFT;
-        if (sc < 0 || sc >= (int)h->scenes.size()) return fail(h, ZMPM_E_HIP, "corrupt particle scene");
-        for (int a = 0; a < 3; a++) {
-            if (p->x) {
-                if constexpr (std::is_same<T, float>::value) {
-                    int X;
-                    std::memcpy(&X, &buf[(PX + a) * cap + s], sizeof(int));
-                    const zmpm_scene_desc& sd = h->scenes[(size_t)sc];
-                    p->x[3 * i + a] = decodePos(X, sd.dx, posBits(sd.domain_nodes));
-                }
-                else
-                    p->x[3 * i + a] = (double)buf[(PX + a) * cap + s];
+    const Dev<T, AccT>& D = devOf<T, AccT>(h);
+    const int64_t n = h->n;
+    if (n == 0) return ZMPM_OK;
+    ExportJobs J {};
+    char* dst[EXP_MAX];
+    size_t row_bytes[EXP_MAX];
+    auto add = [&](void* to, int field, int width, int kind) {
+        if (!to) return;
+        const int j = J.count++;
+        dst[j] = static_cast<char*>(to);
+        J.field[j] = field;
+        J.width[j] = width;
+        J.kind[j] = kind;
+        row_bytes[j] = kind == EXP_MAT ? sizeof(int32_t) : (size_t)width * sizeof(double);
+        J.off[j + 1] = J.off[j] + (kind == EXP_MAT ? (n + 1) / 2 : n * width);
+    };
+    add(p->x, PX, 3, EXP_POS);
+    add(p->v, PV, 3, EXP_PLAIN);
+    add(p->C, PC, 9, EXP_PLAIN);
+    add(p->F, PF, 9, EXP_F);
+    add(p->m, PM, 1, EXP_PLAIN);
+    add(p->V0, PVOL, 1, EXP_PLAIN);
+    add(p->material, 0, 1, EXP_MAT);
+    add(p->d, PD, 1, EXP_PLAIN);
+    add(p->g, PG, 1, EXP_PLAIN);
+    add(p->laplacian, PLAP, 1, EXP_PLAIN);
+    add(p->plastic_state, PYS, 1, EXP_PLAIN);
+    add(p->max_dtilde, PDT, 1, h->desc.implicit_damage ? EXP_PLAIN : EXP_ZERO);
+    add(p->J, PJ, 1, EXP_J);
+    const int64_t words = J.off[J.count];
+    const int64_t chunk = (int64_t)(kSlotBytes / sizeof(double));
+    const int64_t nchunks = (words + chunk - 1) / chunk;
+    const int want = (int)std::min<int64_t>(nchunks, std::min(kMaxSlots, std::max(1, (int)std::thread::hardware_concurrency())));
+    zmpm_status st = downloadSlots(h, std::max(want, 1), (size_t)words * sizeof(double));
+    if (st != ZMPM_OK) return st;
+    *h->dl_bad = 0;
+    k_export_index<T, AccT><<<gridFor(n, WG, 1 << 30), WG, 0, h->stream>>>(D, h->dl_bad);
+    std::atomic<int64_t> next { 0 };
+    std::atomic<int> error { (int)hipSuccess };
+    auto participate = [&](int slot) {
+        if (hipSetDevice(h->desc.device) != hipSuccess) return;
+        zmpm_context::Slot& sl = h->dl_slots[(size_t)slot];
+        for (int64_t c; (c = next.fetch_add(1)) < nchunks && error.load() == (int)hipSuccess;) {
+            const int64_t w0 = c * chunk, w1 = std::min(w0 + chunk, words);
+            k_export<T, AccT><<<gridFor(w1 - w0, WG, 2048), WG, 0, h->stream>>>(D, J, w0, w1, static_cast<double*>(sl.host));
+            hipError_t e = hipGetLastError();
+            if (e == hipSuccess) e = hipEventRecord(sl.done, h->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(sl.done);
+            if (e != hipSuccess) {
+                error.store((int)e);
+                return;
             }
-            if (p->v) p->v[3 * i + a] = (double)buf[(PV + a) * cap + s];
+            if (*h->dl_bad) return; // the caller reports it
+            for (int j = 0; j < J.count; j++) {
+                const int64_t a = std::max(w0, J.off[j]), b = std::min(w1, J.off[j + 1]);
+                if (a >= b) continue;
+                const size_t at = (size_t)(a - J.off[j]) * sizeof(double);
+                const size_t len = std::min((size_t)(b - a) * sizeof(double), (size_t)n * row_bytes[j] - at);
+                std::memcpy(dst[j] + at, static_cast<const char*>(sl.host) + (size_t)(a - w0) * sizeof(double), len);
+            }
         }
-        for (int k = 0; k < 9; k++) {
-            if (p->C) p->C[9 * i + k] = (double)buf[(PC + k) * cap + s];
-            if (p->F)
-                p->F[9 * i + k] = (double)buf[(PF + k) * cap + s]
-                    + (std::is_same<T, float>::value && k % 4 == 0 ? 1.0 : 0.0);
-        }
-        if (p->m) p->m[i] = (double)buf[PM * cap + s];
-        if (p->V0) p->V0[i] = (double)buf[PVOL * cap + s];
-        if (p->material) p->material[i] = mat[s] & PMAT_MAT_MASK;
-        if (p->d) p->d[i] = (double)buf[PD * cap + s];
-        if (p->g) p->g[i] = (double)buf[PG * cap + s];
-        if (p->laplacian) p->laplacian[i] = (double)buf[PLAP * cap + s];
-        if (p->plastic_state) p->plastic_state[i] = (double)buf[PYS * cap + s];
-        if (p->max_dtilde) p->max_dtilde[i] = h->desc.implicit_damage ? (double)buf[PDT * cap + s] : 0.0;
-        if (p->J) p->J[i] = (double)buf[PJ * cap + s] + (std::is_same<T, float>::value ? 1.0 : 0.0);
+    };
+    std::vector<std::thread> threads;
+    try {
+        threads.reserve((size_t)kMaxSlots);
+        for (int k = 1; k < want; k++) threads.emplace_back(participate, k);
     }
+    catch (...) { // fewer participants
+    }
+    participate(0);
+    for (std::thread& t : threads) t.join();
+    if (nchunks == 0) HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (error.load() != (int)hipSuccess)
+        return fail(h, ZMPM_E_HIP, std::string("download: ") + hipGetErrorString((hipError_t)error.load()));
+    if (next.load() < nchunks && !*h->dl_bad) return fail(h, ZMPM_E_HIP, "download: device not available");
+    if (*h->dl_bad) return fail(h, ZMPM_E_HIP, "corrupt particle id or scene table");
     return ZMPM_OK;
 }
 
@@ -1194,6 +1267,11 @@ zmpm_status zmpm_destroy(zmpm_handle h)
     (void)hipSetDevice(h->desc.device);
     freeAll(h);
     for (hipEvent_t e : h->events) (void)hipEventDestroy(e);
+    for (auto& sl : h->dl_slots) {
+        if (sl.host) (void)hipHostFree(sl.host);
+        (void)hipEventDestroy(sl.done);
+    }
+    if (h->dl_bad) (void)hipHostFree(h->dl_bad);
     for (void* q : { h->mats_dev, h->cols_dev, h->colstate_dev, h->scenes_dev, h->regions_dev, h->bfval_dev })
         if (q) (void)hipFree(q);
     if (h->stream) (void)hipStreamDestroy(h->stream);

@@ -3047,6 +3047,79 @@ __global__ __launch_bounds__(WG) void k_extent(Dev<T, AccT> D, int fold, int row
     }
 }
 
+// ------------------------------------------------------------- download
+// Particle fields in the caller's layout: the requested arrays (doubles, rows
+// of 1, 3 or 9; the material indices as int32) one behind the other in 8-byte
+// words, each in upload order.  The host takes them in ranges of words through
+// pinned buffers the kernel writes directly, so a range crosses PCIe once and
+// in its final form: x, v, C, F and d of 1M particles in 4.5 ms, 44 GB/s
+// (94 ms with every field copied as stored and reordered by one host thread), of
+// 10.4M in 43 ms (914 ms); pinned copies reach 57 GB/s here.
+enum : int { EXP_PLAIN = 0, EXP_POS = 1, EXP_F = 2, EXP_J = 3, EXP_MAT = 4, EXP_ZERO = 5 };
+constexpr int EXP_MAX = 13;
+struct ExportJobs {
+    int count;
+    int field[EXP_MAX], width[EXP_MAX], kind[EXP_MAX];
+    int64_t off[EXP_MAX + 1]; // first word of each array, and the end
+};
+
+// Live index of every original index; an id or a scene out of its range raises *bad.
+template <class T, class AccT>
+__global__ __launch_bounds__(WG) void k_export_index(Dev<T, AccT> D, int* bad)
+{
+    const int s = blockIdx.x * WG + threadIdx.x;
+    if (s >= D.n) return;
+    const int id = D.pid[s], sc = sceneOf(D.pmat[s]);
+    if ((unsigned)id < (unsigned)D.n)
+        D.inv[id] = s;
+    else
+        *bad = 1;
+    if ((unsigned)sc >= (unsigned)D.nscenes) *bad = 1;
+}
+
+// Words [w0, w1) of the arrays to out.  A thread takes single words, so a
+// wavefront writes 512 contiguous bytes; the reads of one particle's row go to
+// neighbouring lanes.
+template <class T, class AccT>
+__global__ __launch_bounds__(WG) void k_export(Dev<T, AccT> D, ExportJobs J, int64_t w0, int64_t w1, double* out)
+{
+    constexpr bool F32 = sizeof(T) == 4;
+    int j = 0;
+    for (int64_t w = w0 + (int64_t)blockIdx.x * WG + threadIdx.x; w < w1; w += (int64_t)gridDim.x * WG) {
+        while (w >= J.off[j + 1]) j++; // words of a thread only grow
+        const int l = (int)(w - J.off[j]), width = J.width[j], kind = J.kind[j];
+        if (kind == EXP_MAT) { // two indices a word
+            int m[2] = { 0, 0 };
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                if (2 * l + h < D.n) m[h] = matOf(D.pmat[D.inv[2 * l + h]]);
+            out[w - w0] = __hiloint2double(m[1], m[0]);
+            continue;
+        }
+        const int i = width == 1 ? l : (width == 3 ? l / 3 : l / 9), k = l - width * i;
+        const int s = D.inv[i];
+        const T* src = D.P + (J.field[j] + k) * D.cap;
+        double v = 0.0;
+        if (kind == EXP_POS) {
+            if constexpr (F32) {
+                // (a corrupt scene, which k_export_index reports, reads scene 0's record)
+                const int sc = sceneOf(D.pmat[s]);
+                const SceneDev<T>& sd = D.sc[(unsigned)sc < (unsigned)D.nscenes ? sc : 0];
+                const int X = __float_as_int((float)src[s]);
+                v = X == POS_NAN ? __longlong_as_double(0x7ff8000000000000LL) : (double)X * sd.ddx / (double)(1 << sd.pos_bits);
+            }
+            else
+                v = src[s];
+        }
+        else if (kind != EXP_ZERO) {
+            v = (double)src[s];
+            // the float form keeps F - I and J - 1
+            if (F32 && (kind == EXP_J || (kind == EXP_F && k % 4 == 0))) v += 1.0;
+        }
+        out[w - w0] = v;
+    }
+}
+
 // ------------------------------------------------- implicit damage solve
 // AnisoFractureSimulation::solveDamageSystem (AnisoFractureSimulation.h:435-612)
 // between the grid update and G2P:

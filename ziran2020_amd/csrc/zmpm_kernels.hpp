@@ -224,6 +224,7 @@ struct Dev {
     int* perm;         // sorted position -> live index
     int* sorted_cell;  // sorted position -> dense cell id
     int* spid;         // sorted position -> original index
+    int* inv;          // original index -> live index (download only)
     int* touched;      // per page: 1 if a particle block or its -1 neighbour has particles
     int* page_count;   // per page: particles whose base node is in the page
     int* page_table;   // per page: dense block id or -1
