@@ -855,15 +855,14 @@ __device__ __forceinline__ Mat3<T> loadM(const T* P, int64_t cap, int f, int p)
 template <bool FAST = false>
 __device__ __forceinline__ bool vtauSym(const MatDev<float>& mt, const Mat3<float>& H, float V0, float g, float* S)
 {
-    float t6[6];
+    float t6[6], scale = V0;
     if (mt.model == ZMPM_MODEL_EQUATION_OF_STATE) {
         const float jm1 = H.a[0][0];
-        const float p = V0 * (-mt.bulk * expm1f(-mt.gamma * log1pf(jm1))) * (1.f + jm1);
-        S[0] = S[3] = S[5] = p;
-        S[1] = S[2] = S[4] = 0.f;
-        return false;
+        t6[0] = t6[3] = t6[5] = V0 * (-mt.bulk * expm1f(-mt.gamma * log1pf(jm1))) * (1.f + jm1);
+        t6[1] = t6[2] = t6[4] = 0.f;
+        scale = 1.f;
     }
-    if (mt.model == ZMPM_MODEL_FIXED_COROTATED) {
+    else if (mt.model == ZMPM_MODEL_FIXED_COROTATED) {
         if (corotatedTauH<FAST>(H, mt.mu, mt.lambda, t6)) return true;
     }
     else if (mt.model == ZMPM_MODEL_QR_STABLE_NEO_HOOKEAN) {
@@ -881,7 +880,7 @@ __device__ __forceinline__ bool vtauSym(const MatDev<float>& mt, const Mat3<floa
     else
         neoHookeanTauH(H, mt.mu, mt.lambda, t6);
 #pragma unroll
-    for (int i = 0; i < 6; i++) S[i] = V0 * t6[i];
+    for (int i = 0; i < 6; i++) S[i] = scale * t6[i];
     return false;
 }
 
@@ -2226,8 +2225,8 @@ __device__ __forceinline__ bool damageUpdate(const MatDev<T>& mt, const Mat3<T>&
 // damage update on F_n, then the stress of (F_{n+1}, g_{n+1}) that the next
 // substep's forcesUpdateParticleState would compute, and the next P2G's
 // fixed-point bounds.  One thread per sorted particle (max_slots workgroups of
-// WG particles); the grid velocities of each block segment of the workgroup's
-// particles (block + halo) are staged in LDS first.  Output goes to sorted
+// WG particles); the tiles (block + halo) of the blocks that the workgroup's
+// particles lie in are staged in LDS first, several at a time.  Output goes to sorted
 // position s of the other buffer.
 // Per-particle G2P state carried from the gather to the finish.
 template <class T>
@@ -2276,6 +2275,9 @@ __device__ __forceinline__ void g2pGather(const Dev<T, AccT>& D, const SceneDev<
     const int ly0 = cell >= 0 ? (cell >> B::zbits) & (TL::BY - 1) : base[1] & (TL::BY - 1);
     const int lz0 = cell >= 0 ? cell & (TL::BZ - 1) : base[2] & (TL::BZ - 1);
     T lap = T(0);
+    // x weights of the running node first, moved up by one each time (indexed by
+    // the loop they would live in memory)
+    T xw[3] = { w[0][0], w[0][1], w[0][2] }, xd[3] = { dw[0][0], dw[0][1], dw[0][2] }, xo[3] = { off[0][0], off[0][1], off[0][2] };
 #pragma unroll 1
     for (int i = 0; i < 3; i++) {
         // sums over j of the z-sums: tv = sum wy s0, ty = sum wy (y_j - y_p) s0,
@@ -2330,7 +2332,10 @@ __device__ __forceinline__ void g2pGather(const Dev<T, AccT>& D, const SceneDev<
                 q2 += wy * p1;
             }
         }
-        const T wx = w[0][i], dwx = dw[0][i], wxo = w[0][i] * off[0][i];
+        const T wx = xw[0], dwx = xd[0], wxo = xw[0] * xo[0];
+        xw[0] = xw[1], xw[1] = xw[2];
+        xd[0] = xd[1], xd[1] = xd[2];
+        xo[0] = xo[1], xo[1] = xo[2];
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             A.picV[a] += wx * tv[a];
@@ -2367,8 +2372,8 @@ struct RawG2P {
 // G2P's particle fields in two parts: what the gather needs (position and
 // material word) and what only the finish needs (F, m, V0, d, g, original
 // index, plastic state, J; FLIP: v).  The float form loads the second part
-// after the gather, so it is not live across it: 120 instead of 134 VGPRs, 4
-// wavefronts per SIMD instead of 3 (G2P ~8 % faster); the double form, at 2
+// after the gather, so it is not live across it: 115 VGPRs, 4 wavefronts per
+// SIMD instead of 3 (G2P ~8 % faster); the double form, at 2
 // wavefronts either way, loads both up front.
 template <class T, class AccT>
 __device__ __forceinline__ void loadG2PGather(const Dev<T, AccT>& D, int p, RawG2P<T>& r)
@@ -2554,48 +2559,82 @@ __device__ __forceinline__ bool g2pFinish(const Dev<T, AccT>& D, int s, const Ra
     return rare;
 }
 
-// Grid node records of block b's tile (the block and its forward halo, through
-// the neighbour table) into gt: gt[0] the new velocity and phase field, and
-// with nrec = 2 gt[1] the grid's velocity before the update (FLIP).  A node
-// outside the grid stages zeros.
-template <class T, class AccT>
-__device__ __forceinline__ void stageTile(const Dev<T, AccT>& D, int b, V4<T> (*gt)[Tile<T>::TN], int nrec)
+// Grid node records of the tiles of nt blocks (a block and its forward halo,
+// through the neighbour table) into gt, tile u that of block sb[u]: record 0 the
+// new velocity and phase field, and with NREC = 2 record 1 the grid's velocity
+// before the update (FLIP).  A node outside the grid stages zeros.
+template <class T, class AccT, int NREC>
+__device__ __forceinline__ void stageTiles(const Dev<T, AccT>& D, const int* sb, int nt, V4<T> (*gt)[NREC][Tile<T>::TN])
 {
     using B = Blk<T>;
     using TL = Tile<T>;
     constexpr int NB = TL::NB;
-    // the neighbour table row, read once (a uniform address) and selected per node
-    const int* nb = D.nbr + b * 8;
-    int nbv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) nbv[i] = nb[i];
-    for (int e = threadIdx.x; e < nrec * TL::TN; e += WG) {
-        const int r = e / TL::TN, nd = e - TL::TN * (e / TL::TN);
+    for (int e = threadIdx.x; e < nt * TL::TN; e += WG) {
+        const int u = e / TL::TN, nd = e - TL::TN * (e / TL::TN);
         const int tx = nd / (TL::TY * TL::TZ), ty = (nd / TL::TZ) % TL::TY, tz = nd % TL::TZ;
         const int which = ((tx >= TL::BX) << 2) | ((ty >= TL::BY) << 1) | (tz >= TL::BZ);
-        int tb = nbv[0];
+        const int tb = D.nbr[sb[u] * 8 + which];
+        const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits) | (tz & (TL::BZ - 1));
+        const int64_t node = (int64_t)tb * NB + elem;
 #pragma unroll
-        for (int i = 1; i < 8; i++) tb = which == i ? nbv[i] : tb;
-        V4<T> v { T(0), T(0), T(0), T(0) };
-        if (tb >= 0) {
-            const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits) | (tz & (TL::BZ - 1));
-            const int64_t node = (int64_t)tb * NB + elem;
-            v = nodeRec(r == 0 ? D.newv : D.oldv, node);
+        for (int r = 0; r < NREC; r++) {
+            typedef T Rec __attribute__((ext_vector_type(4)));
+            Rec v = T(0);
+            if (tb >= 0) v = reinterpret_cast<const Rec*>(r == 0 ? D.newv : D.oldv)[node];
+            *reinterpret_cast<Rec*>(&gt[u][r][nd]) = v;
         }
-        gt[r][nd] = v;
     }
 }
+
+// The runs of one block's particles among the workgroup's [lo, hi) (this thread:
+// sorted position s): sb[k] gets the block of run k, *runs (an LDS word) their
+// number; returns the run of s (-1: no particle).  Ends on a barrier.
+template <class T, class AccT>
+__device__ __forceinline__ int blockRuns(const Dev<T, AccT>& D, int lo, int hi, int s, int* sb, int* runs)
+{
+    constexpr int NB = Tile<T>::NB;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool live = s < hi;
+    const int b = live ? ldAt(D.sorted_cell, s) / NB : -1;
+    int prev = __shfl_up(b, 1);
+    if (lane == 0) prev = live && s > lo ? ldAt(D.sorted_cell, s - 1) / NB : -1;
+    const uint64_t heads = __ballot(live && b != prev);
+    if (lane == 0) runs[wv] = __popcll(heads);
+    ldsBarrier();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < WG / 64; w++) {
+        if (w < wv) before += runs[w];
+        all += runs[w];
+    }
+    const int run = before + __popcll(heads & (~0ull >> (63 - lane))) - 1;
+    if (live && b != prev) sb[run] = b;
+    ldsBarrier();
+    if (threadIdx.x == 0) runs[0] = all;
+    ldsBarrier();
+    return live ? run : -1;
+}
+
+// Tiles staged at once by G2P: its 256 particles span one to three blocks where
+// they are dense, and dozens on a surface or in a sparse scene, where staging one
+// block after the other kept a workgroup for up to 135 us (mean 21): each block
+// is a chain of three dependent loads and a pass through the gather.  Eight
+// tiles are 27.6 KB (FP64 36.9 KB, FLIP the same with four): the four (two)
+// workgroups a CU holds by registers fit its LDS.  Measured with the gather and
+// the finish compiled once each (a scene's table by wave-uniform pass and by
+// lane; 115 VGPRs, 18 KB of code less), event-timed, before -> after: 512 particles
+// 30 -> 17 us, 130k FLIP 57 -> 27, 262k FP64 75 -> 47, 1M slab 87 -> 74, 4M
+// two-material column 437 -> 344, 10.4M batched scenes 912 -> 816.
+template <class T, bool FLIP> struct G2PTiles { static constexpr int value = FLIP ? 4 : 8; };
 
 // RR: workgroups take particle segments round-robin over the XCDs instead of
 // XCD by XCD (an autotuner variant; results are the same).
 template <class T, class AccT, bool FLIP, bool RR = false>
-__global__ __launch_bounds__(WG) void k_g2p(Dev<T, AccT> D)
+__global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT> D)
 {
-    using TL = Tile<T>;
-    constexpr int NB = TL::NB;
-    constexpr int NGT = FLIP ? 7 : 4;
-    __shared__ V4<T> gt[(NGT + 3) / 4][TL::TN];
-    __shared__ int seg_end;
+    constexpr int NREC = FLIP ? 2 : 1, NT = G2PTiles<T, FLIP>::value;
+    __shared__ V4<T> gt[NT][NREC][Tile<T>::TN];
+    __shared__ int run_block[WG], runs[WG / 64];
     const int lo = (RR ? (int)blockIdx.x : xcdLocal((int)blockIdx.x, (int)gridDim.x)) * WG;
     const int hi = min(lo + WG, D.n);
     const int t = threadIdx.x, s = lo + t;
@@ -2623,35 +2662,30 @@ __global__ __launch_bounds__(WG) void k_g2p(Dev<T, AccT> D)
     }
     A.lap = T(0);
     const int scene = live ? sceneOf(R.mid) : 0;
-    int seg_lo = lo;
-    while (seg_lo < hi) {
-        const int b = D.sorted_cell[seg_lo] / NB;
-        // LDS-only barriers: the particle loads issued above stay in flight
-        // while the tile is staged
-        ldsBarrier(); // previous segment's gathers done
-        if (t == 0) {
-            const int c = b * NB + NB - 1;
-            seg_end = D.cell_start[c] + D.cell_count[c];
-        }
-        stageTile(D, b, gt, FLIP ? 2 : 1);
+    // LDS-only barriers: the particle loads issued above stay in flight while
+    // the tiles are staged
+    const int run = blockRuns(D, lo, hi, s, run_block, runs), nruns = runs[0];
+    for (int k0 = 0; k0 < nruns; k0 += NT) {
+        if (k0 > 0) ldsBarrier(); // previous tiles' gathers done
+        stageTiles<T, AccT, NREC>(D, run_block + k0, min(NT, nruns - k0), gt);
         ldsBarrier();
-        const int seg_hi = max(seg_lo + 1, min(hi, seg_end));
-        // the segment's particles are in its block's scene (a uniform index)
-        if (live && s >= seg_lo && s < seg_hi) g2pGather<T, AccT, FLIP>(D, D.sc[blockScene(D, b)], gt, R.x, dmg, A);
-        seg_lo = seg_hi;
+        // one pass per scene of the wavefront (one but across two scenes' blocks),
+        // its table read with scalar loads through a wave-uniform index (the same
+        // around the finish would keep both sides' registers live: 175)
+        bool mine = run >= k0 && run < k0 + NT;
+        while (mine) {
+            const int sc = __builtin_amdgcn_readfirstlane(scene);
+            if (scene == sc) {
+                g2pGather<T, AccT, FLIP>(D, D.sc[sc], gt[run - k0], R.x, dmg, A);
+                mine = false;
+            }
+        }
     }
     if (LATE && live) loadG2PFinish<T, AccT, FLIP>(D, s, p, R);
     float bnd[NSC] = { 0.f, 0.f, 0.f, 0.f, 0.f };
     PosT<T> xnew[3] = { 0, 0, 0 };
     bool rare = false;
-    // a wavefront of one scene (all but those across two scenes' blocks) reads
-    // the scene's table with scalar loads through a wave-uniform index
-    const int s_first = __builtin_amdgcn_readfirstlane(scene);
-    if (!__ballot(live && scene != s_first)) {
-        if (live) rare = g2pFinish<T, AccT, FLIP>(D, s, R, D.sc[s_first], A, D.mats[matOf(R.mid)], bnd, xnew);
-    }
-    else if (live)
-        rare = g2pFinish<T, AccT, FLIP>(D, s, R, D.sc[scene], A, D.mats[matOf(R.mid)], bnd, xnew);
+    if (live) rare = g2pFinish<T, AccT, FLIP>(D, s, R, D.sc[scene], A, D.mats[matOf(R.mid)], bnd, xnew);
     // deferred particles to the rare-path queue, one atomic per wavefront
     const uint64_t rm = __ballot(rare);
     if (rm) {
@@ -2909,10 +2943,9 @@ __global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
 template <class T, class AccT>
 __global__ __launch_bounds__(WG) void k_damp_g2p(Dev<T, AccT> D)
 {
-    using TL = Tile<T>;
-    constexpr int NB = TL::NB;
-    __shared__ V4<T> gt[1][TL::TN];
-    __shared__ int seg_end;
+    constexpr int NB = Tile<T>::NB, NT = G2PTiles<T, false>::value;
+    __shared__ V4<T> gt[NT][1][Tile<T>::TN];
+    __shared__ int run_block[WG], runs[WG / 64];
     const int lo = xcdLocal((int)blockIdx.x, (int)gridDim.x) * WG;
     const int hi = min(lo + WG, D.n);
     const int t = threadIdx.x, s = lo + t;
@@ -2939,19 +2972,12 @@ __global__ __launch_bounds__(WG) void k_damp_g2p(Dev<T, AccT> D)
         A.gv[i / 3][i % 3] = T(0);
     }
     A.lap = T(0);
-    int seg_lo = lo;
-    while (seg_lo < hi) {
-        const int b = D.sorted_cell[seg_lo] / NB;
-        __syncthreads(); // previous segment's gathers done
-        if (t == 0) {
-            const int c = b * NB + NB - 1;
-            seg_end = D.cell_start[c] + D.cell_count[c];
-        }
-        stageTile(D, b, gt, 1);
-        __syncthreads();
-        const int seg_hi = max(seg_lo + 1, min(hi, seg_end));
-        if (live && s >= seg_lo && s < seg_hi) g2pGather<T, AccT, false>(D, D.sc[blockScene(D, b)], gt, x, false, A, cell);
-        seg_lo = seg_hi;
+    const int run = blockRuns(D, lo, hi, s, run_block, runs), nruns = runs[0];
+    for (int k0 = 0; k0 < nruns; k0 += NT) {
+        if (k0 > 0) ldsBarrier(); // previous tiles' gathers done
+        stageTiles<T, AccT, 1>(D, run_block + k0, min(NT, nruns - k0), gt);
+        ldsBarrier();
+        if (run >= k0 && run < k0 + NT) g2pGather<T, AccT, false>(D, sd, gt[run - k0], x, false, A, cell);
     }
     float bnd[NSC] = { 0.f, 0.f, 0.f, 0.f, 0.f };
     if (live) {
