@@ -1489,24 +1489,28 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
             }
         }
         ldsBarrier();
-        // ---- flush the tile: one HBM atomic per non-zero node value
-        for (int e = t; e < nq * TL::TN; e += WG) {
-            const int f = e / TL::TN, nd = e - TL::TN * (e / TL::TN);
-            const AccT v = tile[f][nd];
-            if (v == AccT(0)) continue;
-            const int tx = nd / (TL::TY * TL::TZ), ty = (nd / TL::TZ) % TL::TY, tz = nd % TL::TZ;
-            const int which = ((tx >= TL::BX) << 2) | ((ty >= TL::BY) << 1) | (tz >= TL::BZ);
-            const int tb = nbl[which];
-            if (tb < 0) {
-                ovf |= 2;
-                continue;
-            }
+        // ---- flush the tile: one HBM atomic per non-zero node value.  Thread t owns
+        // tile node t in every field, so the node's address is formed once (a loop
+        // over field-major values formed it for each: ~70 instructions a value, a
+        // seventh of the kernel's where blocks are dense and more where they are thin)
+        static_assert(TL::TN <= WG, "one thread per tile node");
+        if (t < TL::TN) {
+            const int tx = t / (TL::TY * TL::TZ), ty = (t / TL::TZ) % TL::TY, tz = t % TL::TZ;
+            const int tb = nbl[((tx >= TL::BX) << 2) | ((ty >= TL::BY) << 1) | (tz >= TL::BZ)];
             const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits) | (tz & (TL::BZ - 1));
-            AccT* dst = D.acc + f * cn + (int64_t)tb * NB + elem;
-            if constexpr (FIXED)
-                atomicAdd((unsigned long long*)dst, (unsigned long long)v);
-            else
-                unsafeAtomicAdd(dst, v);
+            AccT* dst = D.acc + (int64_t)tb * NB + elem;
+#pragma unroll
+            for (int f = 0; f < NGF; f++, dst += cn) {
+                if (f >= nq) break;
+                const AccT v = tile[f][t];
+                if (v == AccT(0)) continue;
+                if (tb < 0)
+                    ovf |= 2;
+                else if constexpr (FIXED)
+                    atomicAdd((unsigned long long*)dst, (unsigned long long)v);
+                else
+                    unsafeAtomicAdd(dst, v);
+            }
         }
     }
     if (ovf & 1) latch(D.counters, ST_OVERFLOW);
