@@ -272,7 +272,8 @@ zmpm_status allocate(zmpm_context* h, int n)
     ALLOC(D.key, cap);
     ALLOC(D.rank, cap);
     ALLOC(D.tmp, cap);
-    ALLOC(D.rare, cap);
+    ALLOC(D.rare, RARE_QUEUES * rareQueueSize((int)((cap + WG - 1) / WG)));
+    ALLOC(D.rare_count, RARE_QUEUES * RARE_STRIDE);
     ALLOC(D.tmpk, cap);
     ALLOC(D.perm, cap);
     ALLOC(D.sorted_cell, cap);
@@ -324,8 +325,8 @@ zmpm_status allocate(zmpm_context* h, int n)
         HIPCHK(h, hipMemsetAsync(D.cg_bar, 0, 4 * sizeof(unsigned), h->stream));
     }
     {
-        // k_rare walks its queue grid-stride: one resident round of workgroups
-        // serves any queue, and an empty one costs a single round of starts
+        // k_rare walks its queues grid-stride: one resident round of workgroups
+        // serves any queue, and empty ones cost a single round of starts
         int occ = 0, cus = 0;
         HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_rare<T, AccT>, WG, 0));
         HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->desc.device));
@@ -343,6 +344,7 @@ zmpm_status allocate(zmpm_context* h, int n)
     HIPCHK(h, hipMemsetAsync(D.spid, 0, cap * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.inv, 0, cap * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.counters, 0, 8 * sizeof(int), h->stream));
+    HIPCHK(h, hipMemsetAsync(D.rare_count, 0, RARE_QUEUES * RARE_STRIDE * sizeof(int), h->stream));
     HIPCHK(h, hipMemsetAsync(D.maxbits, 0, ns * NSC * BOUND_SLOTS * sizeof(unsigned int), h->stream));
     const std::vector<float> ones((size_t)(NSC * ns), 1.f);
     HIPCHK(h, hipMemcpyAsync(D.scales, ones.data(), ones.size() * sizeof(float), hipMemcpyHostToDevice, h->stream));

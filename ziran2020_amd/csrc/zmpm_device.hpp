@@ -280,7 +280,7 @@ __device__ __forceinline__ uint64_t waveInclusiveScan64(uint64_t v)
 // reference's unique 64-bit keys (MpmSimulationBase.cpp:1552).
 
 // counters[] slots
-enum : int { CNT_BLOCKS = 0, CNT_STATUS = 1, CNT_EPOCH = 2, CNT_TICKET = 3, CNT_RARE = 4, CNT_SUPER = 5, CNT_TICKET2 = 6 };
+enum : int { CNT_BLOCKS = 0, CNT_STATUS = 1, CNT_EPOCH = 2, CNT_TICKET = 3, CNT_SUPER = 5, CNT_TICKET2 = 6 };
 
 constexpr int PSCAN_ITEMS = 8;
 constexpr int PSCAN_TILE = WG * PSCAN_ITEMS; // pages per scan tile
@@ -623,8 +623,7 @@ template <class T, class AccT>
 __device__ __forceinline__ void beginStep(const Dev<T, AccT>& D)
 {
     // clock[2 s] = time of the scene's next substep, clock[2 s + 1] = this
-    // substep's t; the rare-path queue of this substep's G2P starts empty
-    if (threadIdx.x == 0) D.counters[CNT_RARE] = 0;
+    // substep's t
     for (int sc = threadIdx.x; sc < D.nscenes; sc += WG) {
         D.clock[2 * sc + 1] = D.clock[2 * sc];
         D.clock[2 * sc] = D.clock[2 * sc] + D.sc[sc].ddt;
@@ -646,6 +645,8 @@ __device__ __forceinline__ void beginStep(const Dev<T, AccT>& D)
 #pragma unroll
         for (int a = 0; a < 3; a++) D.bfval[3 * e + a] = amp * sd.bf_dir[k][a];
     }
+    // the rare-path queues of this substep's G2P start empty
+    if (threadIdx.x < RARE_QUEUES) D.rare_count[threadIdx.x * RARE_STRIDE] = 0;
     if constexpr (!std::is_same<AccT, long long>::value) return;
     // one wavefront per (scene, scale group) over the BOUND_SLOTS slots, which
     // are cleared for this substep's G2P
@@ -2690,14 +2691,14 @@ __global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT>
     PosT<T> xnew[3] = { 0, 0, 0 };
     bool rare = false;
     if (live) rare = g2pFinish<T, AccT, FLIP>(D, s, R, D.sc[scene], A, D.mats[matOf(R.mid)], bnd, xnew);
-    // deferred particles to the rare-path queue, one atomic per wavefront
+    // deferred particles to the workgroup's rare-path queue, one atomic per wavefront
     const uint64_t rm = __ballot(rare);
     if (rm) {
-        const int lane = t & 63, first = __ffsll((unsigned long long)rm) - 1;
+        const int lane = t & 63, first = __ffsll((unsigned long long)rm) - 1, q = (int)blockIdx.x % RARE_QUEUES;
         int at = 0;
-        if (lane == first) at = atomicAdd(&D.counters[CNT_RARE], __popcll(rm));
+        if (lane == first) at = atomicAdd(&D.rare_count[q * RARE_STRIDE], __popcll(rm));
         at = __shfl(at, first);
-        if (rare) stAt(D.rare, at + __popcll(rm & ((1ull << lane) - 1)), s);
+        if (rare) D.rare[(int64_t)q * rareQueueSize(D.max_slots) + at + __popcll(rm & ((1ull << lane) - 1))] = s;
     }
     // binning of the coming substep at the new positions (live index s)
     openPageScan(D);
@@ -2880,19 +2881,31 @@ __device__ __forceinline__ bool plasticMayProject(const MatDev<float>& mt, const
     return n - lim > -(1e-4f * lim + 1e-6f);
 }
 
-// The particles G2P deferred (queued by sorted position): the AnisoMPM damage
+// The particles G2P deferred (queued by sorted position, the queues walked as
+// one list): the AnisoMPM damage
 // update on F_n with its full path (sigma^+, structural tensor) and the stress of
 // (F_{n+1}, g_{n+1}) with every branch of the models, and its force bound.  Runs
 // after k_g2p of the same substep, before the buffers swap.
 template <class T, class AccT>
 __global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
 {
-    const int cnt = D.counters[CNT_RARE];
+    int qn[RARE_QUEUES], cnt = 0;
+#pragma unroll
+    for (int q = 0; q < RARE_QUEUES; q++) {
+        qn[q] = D.rare_count[q * RARE_STRIDE];
+        cnt += qn[q];
+    }
     const int64_t cap = D.cap;
     for (int base = blockIdx.x * WG; base < cnt; base += gridDim.x * WG) {
         float bnd[NSC] = { 0.f, 0.f, 0.f, 0.f, 0.f };
-        const int i = base + threadIdx.x;
-        int s = i < cnt ? ldAt(D.rare, i) : -1;
+        int s = -1, i = base + (int)threadIdx.x;
+        int64_t at = -1;
+#pragma unroll
+        for (int q = 0; q < RARE_QUEUES; q++) {
+            if (i >= 0 && i < qn[q]) at = (int64_t)q * rareQueueSize(D.max_slots) + i;
+            i -= qn[q];
+        }
+        if (at >= 0) s = D.rare[at];
         if ((unsigned)s >= (unsigned)D.n) s = -1;
         int scene = -1;
         if (s >= 0) {

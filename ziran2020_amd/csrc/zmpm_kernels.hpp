@@ -203,6 +203,15 @@ struct SceneDev {
 constexpr int PMAT_SCENE_SHIFT = 8; // material index in bits 0-7, scene above
 constexpr int PMAT_MAT_MASK = 0xff;
 
+// Queues of the particles G2P defers to k_rare: workgroup w appends to queue
+// w % RARE_QUEUES, whose count has a cache line of its own.  With one count for
+// all, its atomics passed one after the other at ~7 ns each: G2P with k_rare took
+// 121 us instead of 77 on 328,509 particles that nearly all yield, 107 instead
+// of 84 on 250,007 (FP64) under damage (16 counts in one line: as slow as one).
+constexpr int RARE_QUEUES = 16, RARE_STRIDE = 32;
+// Entries of a queue: every particle of its workgroups (256 each).
+__host__ __device__ constexpr int64_t rareQueueSize(int wgs) { return (int64_t)((wgs + RARE_QUEUES - 1) / RARE_QUEUES) * 256; }
+
 // Kernel-visible state of one handle.
 template <class T, class AccT>
 struct Dev {
@@ -218,7 +227,8 @@ struct Dev {
     // binning
     uint64_t* key;     // (page << block_bits | elem) per live particle
     int* rank;         // slot inside the particle's page (k_bin)
-    int* rare;         // sorted positions G2P deferred to k_rare (count in counters[4])
+    int* rare;         // sorted positions G2P deferred to k_rare, RARE_QUEUES queues
+    int* rare_count;   // their counts, RARE_STRIDE apart
     int* tmp;          // sorted position -> live index, before the in-block sort
     uint32_t* tmpk;    // the same positions: cell << (32 - block bits) | original index
     int* perm;         // sorted position -> live index
@@ -243,7 +253,7 @@ struct Dev {
     int* nbr;          // [cap_blocks][8] forward neighbour block ids
     int* cell_count;   // [cap_blocks*NB]
     int* cell_start;   // [cap_blocks*NB]
-    int* counters;     // [0] num_blocks, [1] status bits, [2] scan epoch, [3] scan ticket, [4] rare count
+    int* counters;     // [0] num_blocks, [1] status bits, [2] scan epoch, [3] scan ticket
     double* clock;     // per scene: [2 s] time of the next substep, [2 s + 1] time of the running substep
     int cap_blocks;
     int domain;
