@@ -2567,27 +2567,42 @@ __device__ __forceinline__ bool g2pFinish(const Dev<T, AccT>& D, int s, const Ra
 // Grid node records of the tiles of nt blocks (a block and its forward halo,
 // through the neighbour table) into gt, tile u that of block sb[u]: record 0 the
 // new velocity and phase field, and with NREC = 2 record 1 the grid's velocity
-// before the update (FLIP).  A node outside the grid stages zeros.
-template <class T, class AccT, int NREC>
+// before the update (FLIP).  A node outside the grid stages zeros.  Thread t takes
+// node t of every tile, so a node's place is formed once, and the neighbour
+// lookups of all tiles are in flight together, then their records.
+template <class T, class AccT, int NREC, int NT>
 __device__ __forceinline__ void stageTiles(const Dev<T, AccT>& D, const int* sb, int nt, V4<T> (*gt)[NREC][Tile<T>::TN])
 {
     using B = Blk<T>;
     using TL = Tile<T>;
     constexpr int NB = TL::NB;
-    for (int e = threadIdx.x; e < nt * TL::TN; e += WG) {
-        const int u = e / TL::TN, nd = e - TL::TN * (e / TL::TN);
-        const int tx = nd / (TL::TY * TL::TZ), ty = (nd / TL::TZ) % TL::TY, tz = nd % TL::TZ;
-        const int which = ((tx >= TL::BX) << 2) | ((ty >= TL::BY) << 1) | (tz >= TL::BZ);
-        const int tb = D.nbr[sb[u] * 8 + which];
-        const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits) | (tz & (TL::BZ - 1));
-        const int64_t node = (int64_t)tb * NB + elem;
+    typedef T Rec __attribute__((ext_vector_type(4)));
+    static_assert(TL::TN <= WG, "one thread per tile node");
+    const int nd = threadIdx.x;
+    if (nd >= TL::TN) return;
+    const int tx = nd / (TL::TY * TL::TZ), ty = (nd / TL::TZ) % TL::TY, tz = nd % TL::TZ;
+    const int which = ((tx >= TL::BX) << 2) | ((ty >= TL::BY) << 1) | (tz >= TL::BZ);
+    const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits) | (tz & (TL::BZ - 1));
+    int tb[NT];
 #pragma unroll
-        for (int r = 0; r < NREC; r++) {
-            typedef T Rec __attribute__((ext_vector_type(4)));
-            Rec v = T(0);
-            if (tb >= 0) v = reinterpret_cast<const Rec*>(r == 0 ? D.newv : D.oldv)[node];
-            *reinterpret_cast<Rec*>(&gt[u][r][nd]) = v;
-        }
+    for (int u = 0; u < NT; u++) tb[u] = u < nt ? D.nbr[sb[u] * 8 + which] : -1;
+    constexpr int HALF = NT * NREC > 4 ? NT / 2 : NT; // records in registers at once
+#pragma unroll
+    for (int u0 = 0; u0 < NT; u0 += HALF) {
+        if (u0 >= nt) break;
+        Rec v[HALF][NREC];
+#pragma unroll
+        for (int u = 0; u < HALF; u++)
+#pragma unroll
+            for (int r = 0; r < NREC; r++) {
+                v[u][r] = T(0);
+                if (tb[u0 + u] >= 0) v[u][r] = reinterpret_cast<const Rec*>(r == 0 ? D.newv : D.oldv)[(int64_t)tb[u0 + u] * NB + elem];
+            }
+#pragma unroll
+        for (int u = 0; u < HALF; u++)
+            if (u0 + u < nt)
+#pragma unroll
+                for (int r = 0; r < NREC; r++) *reinterpret_cast<Rec*>(&gt[u0 + u][r][nd]) = v[u][r];
     }
 }
 
@@ -2672,7 +2687,7 @@ __global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT>
     const int run = blockRuns(D, lo, hi, s, run_block, runs), nruns = runs[0];
     for (int k0 = 0; k0 < nruns; k0 += NT) {
         if (k0 > 0) ldsBarrier(); // previous tiles' gathers done
-        stageTiles<T, AccT, NREC>(D, run_block + k0, min(NT, nruns - k0), gt);
+        stageTiles<T, AccT, NREC, NT>(D, run_block + k0, min(NT, nruns - k0), gt);
         ldsBarrier();
         // one pass per scene of the wavefront (one but across two scenes' blocks),
         // its table read with scalar loads through a wave-uniform index (the same
@@ -2992,7 +3007,7 @@ __global__ __launch_bounds__(WG) void k_damp_g2p(Dev<T, AccT> D)
     const int run = blockRuns(D, lo, hi, s, run_block, runs), nruns = runs[0];
     for (int k0 = 0; k0 < nruns; k0 += NT) {
         if (k0 > 0) ldsBarrier(); // previous tiles' gathers done
-        stageTiles<T, AccT, 1>(D, run_block + k0, min(NT, nruns - k0), gt);
+        stageTiles<T, AccT, 1, NT>(D, run_block + k0, min(NT, nruns - k0), gt);
         ldsBarrier();
         if (run >= k0 && run < k0 + NT) g2pGather<T, AccT, false>(D, sd, gt[run - k0], x, false, A, cell);
     }
