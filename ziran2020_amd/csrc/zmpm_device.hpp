@@ -645,8 +645,6 @@ __device__ __forceinline__ void beginStep(const Dev<T, AccT>& D)
 #pragma unroll
         for (int a = 0; a < 3; a++) D.bfval[3 * e + a] = amp * sd.bf_dir[k][a];
     }
-    // the rare-path queues of this substep's G2P start empty
-    if (threadIdx.x < RARE_QUEUES) D.rare_count[threadIdx.x * RARE_STRIDE] = 0;
     if constexpr (!std::is_same<AccT, long long>::value) return;
     // one wavefront per (scene, scale group) over the BOUND_SLOTS slots, which
     // are cleared for this substep's G2P
@@ -1264,6 +1262,9 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     const int nq = DAMP ? GFO : (dmg ? NGF : GPF);
     const int64_t cap = D.cap, cn = D.cap_nodes;
     const int nblocks = D.counters[0];
+    // the rare-path queues of this substep's G2P start empty (in k_scatter the
+    // address took its SGPRs past the 96 that 8 wavefronts per SIMD have: 4 % slower)
+    if (!DAMP && blockIdx.x == 0 && t < RARE_QUEUES) D.rare_count[t * RARE_STRIDE] = 0;
 
     // in-block order of this workgroup's blocks first (a loop of its own, so
     // its registers are free again for the scatter)
