@@ -34,3 +34,18 @@ def test_deferred_particles(gpu, oracle, precision, n, every):
         assert normwise(g[k], o[k]) < TOL[precision], k
     if n > 1:
         assert (o["plastic_state"][::every] > 2.0).any()
+
+
+# deferred particles beside the next substep's page scan (a run: graphs of eight and two, an
+# odd last substep) against each substep as a call of its own
+@pytest.mark.gpu
+@pytest.mark.parametrize("steps", (1, 2, 3, 11))
+def test_run_is_its_substeps(gpu, steps):
+    sc = yielding(4353, 7)
+    a = run(gpu, sc, A.PREC_FP32, steps).download()
+    sim = sc.make(gpu, A.PREC_FP32)
+    for k in range(steps):
+        sim.substep(sc.dt, sc.t0 + k * sc.dt)
+    b = sim.download()
+    for k in ("x", "v", "C", "F", "plastic_state"):
+        assert np.array_equal(a[k], b[k]), k

@@ -145,6 +145,7 @@ struct zmpm_context {
     int p2g_wgs = 2048, grid_wgs = 2048, prep_wgs = 8192;
     bool p2g_wgs_env = false; // P2G workgroups set by ZMPM_P2G_WGS
     int rare_wgs = 1024; // k_rare's grid: its workgroups resident at once on the device
+    bool rare_pending = false; // inside a call: the last G2P's deferred particles wait for the next page scan
     int variant = 0; // compiled kernel variants (VARIANT_* bits), none changes a result
     bool launch_set = false; // configured by zmpm_set_launch_config or the autotuner
 };
@@ -582,17 +583,25 @@ void launchP2G(zmpm_context* h, const Dev<T, AccT>& D, hipStream_t st)
 }
 
 // The kernels of one substep stage (zmpm_stage_id); launchStep runs all five.
+// more: another substep follows in this call, before anything else.
 template <class T, class AccT>
-void launchStage(zmpm_context* h, int stage)
+void launchStage(zmpm_context* h, int stage, bool more = false)
 {
     Dev<T, AccT>& D = devOf<T, AccT>(h);
     hipStream_t st = h->stream;
     switch (stage) {
     case ZMPM_STAGE_SORT: {
         const int gp = gridFor(D.n, WG, 1 << 30);
-        // the touched super pages in order, then the scan of their pages
-        k_super_scan<T, AccT><<<(int)((D.num_super + PSCAN_TILE - 1) / PSCAN_TILE), WG, 0, st>>>(D);
-        k_page_scan<T, AccT><<<(int)std::min<int64_t>(D.num_super, kPageScanWgs), WG, 0, st>>>(D);
+        // a large domain's touched super pages in order, then the scan of their pages,
+        // with the particles the G2P before it in this call deferred
+        if (D.num_super > PSCAN_TILE)
+            k_super_scan<T, AccT><<<(int)((D.num_super + PSCAN_TILE - 1) / PSCAN_TILE), WG, 0, st>>>(D);
+        const int scan = (int)std::min<int64_t>(D.num_super, kPageScanWgs);
+        if (h->rare_pending)
+            k_page_scan_rare<T, AccT><<<scan + std::min(D.max_slots, h->rare_wgs), WG, 0, st>>>(D, scan);
+        else
+            k_page_scan<T, AccT><<<scan, WG, 0, st>>>(D);
+        h->rare_pending = false;
         const int prep = (int)std::min<int64_t>(D.cap_blocks, h->prep_wgs);
         k_scatter<T, AccT><<<gp + prep + 1, WG, 0, st>>>(D, gp, prep);
         break;
@@ -628,13 +637,16 @@ void launchStage(zmpm_context* h, int stage)
             k_g2p<T, AccT, false, true><<<D.max_slots, WG, 0, st>>>(D);
         else
             k_g2p<T, AccT, false><<<D.max_slots, WG, 0, st>>>(D);
-        k_rare<T, AccT><<<std::min(D.max_slots, h->rare_wgs), WG, 0, st>>>(D);
+        // the deferred particles now, or beside the page scan of the call's next
+        // substep (the damping passes need them now)
+        const int damping = D.flip ? h->desc.pic_damping_iteration : h->desc.rpic_damping_iteration;
+        h->rare_pending = more && damping == 0;
+        if (!h->rare_pending) k_rare<T, AccT><<<std::min(D.max_slots, h->rare_wgs), WG, 0, st>>>(D);
         std::swap(D.P, D.Q);
         std::swap(D.pid, D.qid);
         std::swap(D.pmat, D.qmat);
         // RPIC / PIC damping passes (MpmSimulationBase.cpp:318-348) on the moved
         // particles, through this substep's binning
-        const int damping = D.flip ? h->desc.pic_damping_iteration : h->desc.rpic_damping_iteration;
         constexpr bool FIXED = std::is_same<AccT, long long>::value;
         for (int it = 0; it < damping; it++) {
             k_damp_prep<T, AccT><<<gridFor(D.cap_nodes, WG, h->prep_wgs) + (FIXED ? 1 : 0), WG, 0, st>>>(D);
@@ -652,11 +664,11 @@ void launchStage(zmpm_context* h, int stage)
 // One substep: the five stages, with the timing events between them when given
 // (events 0..5 bracket sort, P2G, grid update, damage solve, G2P).
 template <class T, class AccT>
-void launchStep(zmpm_context* h, hipEvent_t* ev)
+void launchStep(zmpm_context* h, hipEvent_t* ev, bool more)
 {
     for (int stage = ZMPM_STAGE_SORT; stage <= ZMPM_STAGE_G2P; stage++) {
         if (ev) (void)hipEventRecord(ev[stage], h->stream);
-        launchStage<T, AccT>(h, stage);
+        launchStage<T, AccT>(h, stage, more && !ev);
     }
     if (ev) (void)hipEventRecord(ev[5], h->stream);
 }
@@ -1485,9 +1497,9 @@ static zmpm_status graphFor(zmpm_handle h, int n, hipGraphExec_t* out)
         return fail(h, ZMPM_E_HIP, "hipStreamBeginCapture");
     for (int k = 0; k < n; k++) {
         if (h->fp32)
-            launchStep<float, long long>(h, nullptr);
+            launchStep<float, long long>(h, nullptr, k + 1 < n);
         else
-            launchStep<double, double>(h, nullptr);
+            launchStep<double, double>(h, nullptr, k + 1 < n);
     }
     if (hipStreamEndCapture(h->stream, &graph) != hipSuccess) return fail(h, ZMPM_E_HIP, "hipStreamEndCapture");
     hipGraphExec_t exec = nullptr;
@@ -1560,9 +1572,9 @@ static zmpm_status runSteps(zmpm_handle h, int32_t steps, const double* dt, cons
     for (; s < steps; s++) {
         if (h->timing) ev = &h->events[(size_t)s * (kTimedGroups + 1)];
         if (h->fp32)
-            launchStep<float, long long>(h, ev);
+            launchStep<float, long long>(h, ev, s + 1 < steps);
         else
-            launchStep<double, double>(h, ev);
+            launchStep<double, double>(h, ev, s + 1 < steps);
     }
     h->stepped = true;
     hipError_t e = hipGetLastError();

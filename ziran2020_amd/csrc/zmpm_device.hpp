@@ -431,8 +431,8 @@ __device__ __forceinline__ uint64_t blockExclusiveScan(uint64_t mine, uint64_t* 
     return off + inc - mine;
 }
 
-// Compaction of the touched super pages in index order (one tile of
-// PSCAN_TILE super pages per workgroup, tiles in ticket order): super_list
+// Compaction of the touched super pages of a large domain in index order (one tile
+// of PSCAN_TILE super pages per workgroup, tiles in ticket order): super_list
 // and their count (CNT_SUPER); the flags are cleared.  Its last tile also
 // zeroes the block count, which the page scan sets when any page is active.
 template <class T, class AccT>
@@ -492,23 +492,47 @@ __global__ __launch_bounds__(WG) void k_super_scan(Dev<T, AccT> D)
 // for the next substep.  Pages of untouched super pages keep stale table
 // entries, which nothing reads: every page a particle or a block's neighbour
 // lookup names was touched.
+// Where the super pages are one tile of flags (domains up to 512 nodes per axis in
+// the float form), every workgroup lists the touched ones itself, which is
+// cheaper than k_super_scan's launch (sort stage of 512 particles 16.8 -> 14.0 us, of the
+// 1M slab 28.0 -> 25.6 us); P2G then clears the flags.
 template <class T, class AccT>
-__global__ __launch_bounds__(WG) void k_page_scan(Dev<T, AccT> D)
+__device__ __forceinline__ void pageScan(const Dev<T, AccT>& D)
 {
     __shared__ int s_tile;
     __shared__ uint64_t s_wsum[WG / 64];
     __shared__ uint64_t s_prefix;
+    __shared__ int s_list[PSCAN_TILE];
     const int t = threadIdx.x, wv = t >> 6;
     const int64_t np = D.num_pages;
-    const int ntiles = D.counters[CNT_SUPER];
     const unsigned epoch = (unsigned)D.counters[CNT_EPOCH];
+    const bool own = D.num_super <= PSCAN_TILE;
+    int ntiles;
+    if (own) {
+        uint32_t fl[PSCAN_ITEMS];
+        uint64_t mine = 0, total = 0;
+#pragma unroll
+        for (int k = 0; k < PSCAN_ITEMS; k++) {
+            const int sp = t * PSCAN_ITEMS + k;
+            fl[k] = sp < (int)D.num_super && D.super_touched[sp] != 0;
+            mine += fl[k];
+        }
+        int at = (int)blockExclusiveScan(mine, s_wsum, &total);
+#pragma unroll
+        for (int k = 0; k < PSCAN_ITEMS; k++)
+            if (fl[k]) s_list[at++] = t * PSCAN_ITEMS + k;
+        ntiles = (int)total;
+        if (ntiles == 0 && blockIdx.x == 0 && t == 0) D.counters[CNT_BLOCKS] = 0;
+    }
+    else
+        ntiles = D.counters[CNT_SUPER];
     for (;;) {
         if (t == 0) s_tile = atomicAdd(&D.counters[CNT_TICKET], 1);
         __syncthreads();
         const int tile = s_tile;
         __syncthreads(); // s_tile read by every thread before the next ticket
         if (tile >= ntiles) return;
-        const int64_t base = (int64_t)D.super_list[tile] * PSCAN_TILE + (int64_t)t * PSCAN_ITEMS;
+        const int64_t base = (int64_t)(own ? s_list[tile] : D.super_list[tile]) * PSCAN_TILE + (int64_t)t * PSCAN_ITEMS;
         uint32_t fl[PSCAN_ITEMS], ct[PSCAN_ITEMS];
         uint64_t mine = 0;
 #pragma unroll
@@ -559,6 +583,12 @@ __global__ __launch_bounds__(WG) void k_page_scan(Dev<T, AccT> D)
         }
         __syncthreads(); // s_wsum and s_prefix free for the next tile
     }
+}
+
+template <class T, class AccT>
+__global__ __launch_bounds__(WG) void k_page_scan(Dev<T, AccT> D)
+{
+    pageScan(D);
 }
 
 // Eigen's Quaternion::toRotationMatrix of q = (w, x, y, z), row-major.
@@ -1265,6 +1295,10 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     // the rare-path queues of this substep's G2P start empty (in k_scatter the
     // address took its SGPRs past the 96 that 8 wavefronts per SIMD have: 4 % slower)
     if (!DAMP && blockIdx.x == 0 && t < RARE_QUEUES) D.rare_count[t * RARE_STRIDE] = 0;
+    // and so do the super pages' flags, which every workgroup of the page scan read
+    // (a larger domain's are cleared by k_super_scan)
+    if (!DAMP && D.num_super <= PSCAN_TILE)
+        for (int i = (int)blockIdx.x * WG + t; i < (int)D.num_super; i += (int)gridDim.x * WG) D.super_touched[i] = 0;
 
     // in-block order of this workgroup's blocks first (a loop of its own, so
     // its registers are free again for the scatter)
@@ -2902,8 +2936,10 @@ __device__ __forceinline__ bool plasticMayProject(const MatDev<float>& mt, const
 // update on F_n with its full path (sigma^+, structural tensor) and the stress of
 // (F_{n+1}, g_{n+1}) with every branch of the models, and its force bound.  Runs
 // after k_g2p of the same substep, before the buffers swap.
+// P and Q: the live and output buffers of that G2P, qmat its output material words;
+// workgroup wg of nwg.
 template <class T, class AccT>
-__global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
+__device__ __forceinline__ void rareParticles(const Dev<T, AccT>& D, T* P, T* Q, const int* qmat, int wg, int nwg)
 {
     int qn[RARE_QUEUES], cnt = 0;
 #pragma unroll
@@ -2912,7 +2948,7 @@ __global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
         cnt += qn[q];
     }
     const int64_t cap = D.cap;
-    for (int base = blockIdx.x * WG; base < cnt; base += gridDim.x * WG) {
+    for (int base = wg * WG; base < cnt; base += nwg * WG) {
         float bnd[NSC] = { 0.f, 0.f, 0.f, 0.f, 0.f };
         int s = -1, i = base + (int)threadIdx.x;
         int64_t at = -1;
@@ -2927,42 +2963,62 @@ __global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
         if (s >= 0) {
             int p = ldAt(D.perm, s);
             if ((unsigned)p >= (unsigned)D.n) p = 0;
-            const int pm = ldAt(D.qmat, s);
+            const int pm = ldAt(qmat, s);
             scene = sceneOf(pm);
             const SceneDev<T>& sd = D.sc[scene];
             const MatDev<T>& mt = D.mats[matOf(pm)];
             const bool dmg = D.any_damage && mt.has_damage;
-            T d = ldAt(D.P + PD * cap, p), g = ldAt(D.P + PG * cap, p);
+            T d = ldAt(P + PD * cap, p), g = ldAt(P + PG * cap, p);
             if (dmg && !D.implicit && phaseFieldModel(mt.model)) {
-                const Mat3<T> F = loadM(D.P, cap, PF, p); // F_n (FP32 form: H)
-                damageUpdate<T, false>(mt, F, ldAt(D.Q + PLAP * cap, s), sd.dt, d, g);
-                stAt(D.Q + PD * cap, s, d);
-                stAt(D.Q + PG * cap, s, g);
+                const Mat3<T> F = loadM(P, cap, PF, p); // F_n (FP32 form: H)
+                damageUpdate<T, false>(mt, F, ldAt(Q + PLAP * cap, s), sd.dt, d, g);
+                stAt(Q + PD * cap, s, d);
+                stAt(Q + PG * cap, s, g);
             }
-            Mat3<T> Fn = loadM(D.Q, cap, PF, s);
+            Mat3<T> Fn = loadM(Q, cap, PF, s);
             T ys = T(0);
             if (mt.plasticity) {
-                ys = ldAt(D.Q + PYS * cap, s);
+                ys = ldAt(Q + PYS * cap, s);
                 const bool changed = mt.plasticity == ZMPM_PLASTICITY_VON_MISES_STVK_HENCKY ? vonMisesProject(mt, Fn, ys)
                     : mt.plasticity == ZMPM_PLASTICITY_DRUCKER_PRAGER_STVK_HENCKY             ? druckerPragerProject(mt, Fn, ys)
                                                                                              : snowProject(mt, Fn, ys);
                 if (changed) {
 #pragma unroll
-                    for (int k = 0; k < 9; k++) stAt(D.Q + (PF + k) * cap, s, Fn.a[k / 3][k % 3]);
-                    stAt(D.Q + PYS * cap, s, ys);
+                    for (int k = 0; k < 9; k++) stAt(Q + (PF + k) * cap, s, Fn.a[k / 3][k % 3]);
+                    stAt(Q + PYS * cap, s, ys);
                 }
             }
             T S[6];
             if (D.fj_solve_j && mt.fj)
-                fjSolveJStress(mt, false, ldAt(D.Q + PVOL * cap, s), ldAt(D.Q + PJ * cap, s), S);
+                fjSolveJStress(mt, false, ldAt(Q + PVOL * cap, s), ldAt(Q + PJ * cap, s), S);
             else
-                vtauSym<false>(mt, Fn, ldAt(D.Q + PVOL * cap, s) * snowScale(mt, ys), g, S);
+                vtauSym<false>(mt, Fn, ldAt(Q + PVOL * cap, s) * snowScale(mt, ys), g, S);
 #pragma unroll
-            for (int k = 0; k < 6; k++) stAt(D.Q + (PS + k) * cap, s, S[k]);
+            for (int k = 0; k < 6; k++) stAt(Q + (PS + k) * cap, s, S[k]);
             if constexpr (std::is_same<AccT, long long>::value) forceBounds(bnd, S, dmg ? d : T(0), sd.odx, D.any_damage != 0);
         }
         if constexpr (std::is_same<AccT, long long>::value) writeBounds(D.maxbits, bnd, scene);
     }
+}
+
+template <class T, class AccT>
+__global__ __launch_bounds__(WG) void k_rare(Dev<T, AccT> D)
+{
+    rareParticles(D, D.P, D.Q, D.qmat, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// Between two substeps of one call: the page scan of the second (workgroups
+// [0, scan_wgs)) beside the deferred particles of the first, whose output buffers
+// are the live ones by now.  Neither reads what the other writes, and as launches of
+// their own the deferred ones are a serial 10 us and more (substep of 16 small scenes
+// 106 -> 97 us, of 328,509 particles that begin to yield 151 -> 142 us).
+template <class T, class AccT>
+__global__ __launch_bounds__(WG) void k_page_scan_rare(Dev<T, AccT> D, int scan_wgs)
+{
+    if ((int)blockIdx.x < scan_wgs)
+        pageScan(D);
+    else
+        rareParticles(D, D.Q, D.P, D.pmat, (int)blockIdx.x - scan_wgs, (int)gridDim.x - scan_wgs);
 }
 
 // Damping pass G2P, gridToParticles(0) (MpmSimulationBase.cpp:328, 344) with
