@@ -430,6 +430,9 @@ void refreshTables(zmpm_context* h)
     while ((1 << rs) < h->region) rs++;
     D.region_shift = rs;
     D.any_damage = h->any_damage ? 1 : 0;
+    for (uint64_t& w : D.damage_mats) w = 0;
+    for (size_t i = 0; i < h->mats.size(); i++)
+        if (h->mats[i].has_damage) D.damage_mats[i >> 6] |= 1ull << (i & 63);
     D.any_plastic = 0;
     D.any_fj = 0;
     for (const auto& m : h->mats) {

@@ -275,6 +275,7 @@ struct Dev {
     double* bfval;       // [nscenes][MAX_BODY_FORCES][3] body forces at the running substep's time
     int num_cols;
     int any_damage;
+    uint64_t damage_mats[4]; // bit m: material m carries the phase field
     int any_plastic;
     int any_fj;        // some material is FJ-mixed: G2P carries J
     int fj_solve_j;    // FJMixedMpmForceHelper::state == SOLVE_J
