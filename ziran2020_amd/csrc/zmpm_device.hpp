@@ -1175,7 +1175,11 @@ __device__ __forceinline__ int uniformBlockScene(const Dev<T, AccT>& D, int b)
     using B = Blk<T>;
     uint32_t Bx, By, Bz;
     blockOfPage<T>((uint32_t)uniformAt(D.block_page, b), Bx, By, Bz);
-    return max(0, sceneOfNode(D, Bx << B::xbits, By << B::ybits, Bz << B::zbits));
+    const uint32_t rd = (uint32_t)D.region_dim;
+    const uint32_t rx = (Bx << B::xbits) >> D.region_shift, ry = (By << B::ybits) >> D.region_shift,
+                   rz = (Bz << B::zbits) >> D.region_shift;
+    if (rx >= rd || ry >= rd || rz >= rd) return 0;
+    return max(0, uniformAt(D.region_scene, (int)((rx * rd + ry) * rd + rz)));
 }
 
 // Block-local LDS tile geometry: a block of BX x BY x BZ nodes plus the +2
@@ -1372,27 +1376,25 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     int pn = 0;
     auto liveAt = [&](int s) { return DAMP ? s : ldAt(D.perm, s); };
     // cell ranges and neighbour table of the workgroup's next block, loaded a
-    // block ahead (thread t < NB: cell t; threads 64..71: neighbour t - 64)
-    int ns = 0, ne = 0, nn = -1;
+    // block ahead (thread t < NB: start and count of cell t; threads 64..71:
+    // neighbour t - 64) and combined at their use (summed here, each wait for them
+    // was one for all prefetches, and the sum lived in scratch memory)
+    int n0 = 0, n1 = 0;
     auto fetchBlock = [&](int bb) {
         if (bb >= nblocks) return;
-        if (t < NB) {
-            const int c = bb * NB + t;
-            ns = D.cell_start[c];
-            ne = ns + D.cell_count[c];
-        }
-        else if (t >= 64 && t < 72)
-            nn = D.nbr[bb * 8 + t - 64];
+        const int* from = t < NB ? D.cell_start + (int64_t)bb * NB + t : D.nbr + (int64_t)bb * 8 + (t & 7);
+        n0 = *from;
+        n1 = D.cell_count[(int64_t)bb * NB + (t & (NB - 1))];
     };
     fetchBlock(wgl);
     for (int b = wgl; b < nblocks; b += gridDim.x) {
         ldsBarrier(); // previous block flushed
         if (t < NB) {
-            cs[t] = ns;
-            ce[t] = ne;
+            cs[t] = n0;
+            ce[t] = n0 + n1;
         }
         else if (t >= 64 && t < 72)
-            nbl[t - 64] = nn;
+            nbl[t - 64] = n0;
         const int bn = b + (int)gridDim.x;
         fetchBlock(bn);
         ldsBarrier();
@@ -1473,8 +1475,8 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
             }
             // the next block's particle range, for the prefetch of its first chunk
             if (sizeof(T) == 4 && hi == be && bn < nblocks) {
-                if (t == 0) nxr[0] = ns;
-                if (t == NB - 1) nxr[1] = ne;
+                if (t == 0) nxr[0] = n0;
+                if (t == NB - 1) nxr[1] = n0 + n1;
             }
             ldsBarrier();
             // float form: prefetch the next chunk of this block, or after its last
