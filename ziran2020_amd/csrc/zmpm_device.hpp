@@ -1314,9 +1314,13 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     __shared__ V4<T> q[7][CH];
     __shared__ T wl[4][CH][3];
     __shared__ AccT tile[NGF][TL::TN];
-    __shared__ int cs[NB], ce[NB], cl[NB];
+    __shared__ int cl[NB];
     __shared__ int hist[NB], cur[NB], cst[NB];
-    __shared__ int ncl, nbl[8], nxr[2];
+    __shared__ int ncl;
+    // cell ranges and neighbours of the block in work and of the one after it
+    __shared__ struct {
+        int cs[NB], ce[NB], nbl[8];
+    } blk[2];
     // the in-block sort stages (key, live index) in the payload area and the
     // grouped copy in the tile area, both free until the block's first chunk
     constexpr int SA = (int)(sizeof(q) / 8), SB = (int)(sizeof(tile) / 8);
@@ -1375,30 +1379,47 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     // chunk ahead of its fields' loads
     int pn = 0;
     auto liveAt = [&](int s) { return DAMP ? s : ldAt(D.perm, s); };
-    // cell ranges and neighbour table of the workgroup's next block, loaded a
-    // block ahead (thread t < NB: start and count of cell t; threads 64..71:
-    // neighbour t - 64) and combined at their use (summed here, each wait for them
+    // of the chunk that begins at lo: this block's (up to be), or the next block's first
+    auto liveAfter = [&](int lo, int be, int ns, int ne, int none) {
+        const int s = (lo < be ? lo : ns) + pt;
+        return s < (lo < be ? be : ne) ? liveAt(s) : none;
+    };
+    // cell ranges and neighbour table of the workgroup's blocks, loaded two blocks
+    // ahead (thread t < NB: start and count of cell t; threads 64..71:
+    // neighbour t - 64), in LDS one block ahead, and combined at their use (summed here, each wait for them
     // was one for all prefetches, and the sum lived in scratch memory)
     int n0 = 0, n1 = 0;
     auto fetchBlock = [&](int bb) {
         if (bb >= nblocks) return;
-        const int* from = t < NB ? D.cell_start + (int64_t)bb * NB + t : D.nbr + (int64_t)bb * 8 + (t & 7);
-        n0 = *from;
-        n1 = D.cell_count[(int64_t)bb * NB + (t & (NB - 1))];
+        if (t < 64) {
+            n0 = ldAt(D.cell_start, bb * NB + (t & (NB - 1)));
+            n1 = ldAt(D.cell_count, bb * NB + (t & (NB - 1)));
+        }
+        else
+            n0 = ldAt(D.nbr, bb * 8 + (t & 7));
     };
-    fetchBlock(wgl);
-    for (int b = wgl; b < nblocks; b += gridDim.x) {
-        ldsBarrier(); // previous block flushed
+    auto keepBlock = [&](int k) {
         if (t < NB) {
-            cs[t] = n0;
-            ce[t] = n0 + n1;
+            blk[k].cs[t] = n0;
+            blk[k].ce[t] = n0 + n1;
         }
         else if (t >= 64 && t < 72)
-            nbl[t - 64] = n0;
+            blk[k].nbl[t - 64] = n0;
+    };
+    fetchBlock(wgl);
+    keepBlock(0);
+    fetchBlock(wgl + (int)gridDim.x);
+    int par = 0;
+    for (int b = wgl; b < nblocks; b += gridDim.x, par ^= 1) {
+        ldsBarrier(); // previous block flushed
         const int bn = b + (int)gridDim.x;
-        fetchBlock(bn);
+        keepBlock(par ^ 1);
+        fetchBlock(bn + (int)gridDim.x);
         ldsBarrier();
+        const int *const cs = blk[par].cs, *const ce = blk[par].ce, *const nbl = blk[par].nbl;
         const int bs = cs[0], be = ce[NB - 1];
+        // the next block's particles
+        const int ns = blk[par ^ 1].cs[0], ne = bn < nblocks ? blk[par ^ 1].ce[NB - 1] : ns;
         if (be <= bs) continue; // halo-only block
         for (int e = t; e < nq * TL::TN; e += WG) (&tile[0][0])[e] = AccT(0);
         // the block's scene: its dx and fixed-point scales
@@ -1409,11 +1430,12 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
         for (int lo = bs; lo < be; lo += CH) {
             const int hi = min(lo + CH, be);
             ldsBarrier(); // previous chunk's phase B done with the payload
+            if (SPLIT && lo == bs) pn = liveAfter(hi, be, ns, ne, pn);
             // ---- phase A: payload of particle lo + pt from the prefetched fields:
             // its B-spline weights (doW) and its momentum, affine and stress terms (doM)
             if (pt < CH && lo + pt < hi) {
                 if (!have) loadP2G<T, AccT, DAMP>(D, lo > bs ? pn : liveAt(lo + pt), dmg, raw, !doM);
-                if (hi + pt < be && (lo == bs || !SPLIT)) pn = liveAt(hi + pt);
+                if (!SPLIT && hi + pt < be) pn = liveAt(hi + pt);
                 T d0s[3], xb[3];
                 int base[3];
 #pragma unroll
@@ -1473,26 +1495,17 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
                 if (act) cl[__popcll(m & ((1ull << t) - 1))] = t;
                 if (t == 0) ncl = __popcll(m);
             }
-            // the next block's particle range, for the prefetch of its first chunk
-            if (sizeof(T) == 4 && hi == be && bn < nblocks) {
-                if (t == 0) nxr[0] = n0;
-                if (t == NB - 1) nxr[1] = n0 + n1;
-            }
             ldsBarrier();
             // float form: prefetch the next chunk of this block, or after its last
             // chunk the first chunk of the next block, while phase B runs (the
             // double form keeps its registers for phase B)
             have = false;
             if (sizeof(T) == 4) {
-                if (hi + pt < be) {
+                if ((hi < be ? hi : ns) + pt < (hi < be ? be : ne)) {
                     loadP2G<T, AccT, DAMP>(D, pn, dmg, raw, !doM);
                     have = true;
-                    if (hi + CH + pt < be) pn = liveAt(hi + CH + pt);
                 }
-                else if (hi == be && bn < nblocks && nxr[0] + pt < nxr[1]) {
-                    loadP2G<T, AccT, DAMP>(D, liveAt(nxr[0] + pt), dmg, raw, !doM);
-                    have = true;
-                }
+                if (hi < be) pn = liveAfter(hi + CH, be, ns, ne, pn);
             }
             // ---- phase B: lanes = (sub-lane, cell, i, j); R sub-lanes share a column
             const int per = ncl * 9;
