@@ -418,6 +418,7 @@ void refreshTables(zmpm_context* h)
 {
     Dev<T, AccT>& D = devOf<T, AccT>(h);
     D.mats = (const MatDev<T>*)h->mats_dev;
+    D.num_mats = (int)h->mats.size();
     D.cols = (const ColDev*)h->cols_dev;
     D.colstate = (ColState*)h->colstate_dev;
     D.num_cols = (int)colliderCount(h);
@@ -585,6 +586,19 @@ void launchP2G(zmpm_context* h, const Dev<T, AccT>& D, hipStream_t st)
         k_p2g<T, AccT, P2G_STD><<<wgs, WG, 0, st>>>(D);
 }
 
+// G2P: the FLIP form, or the standard form with its particle segments taken as the
+// launch configuration selects.
+template <class T, class AccT, bool FEW>
+void launchG2P(zmpm_context* h, const Dev<T, AccT>& D, hipStream_t st)
+{
+    if (D.flip)
+        k_g2p<T, AccT, true, false, FEW><<<D.max_slots, WG, 0, st>>>(D);
+    else if (h->variant & VARIANT_G2P_RR)
+        k_g2p<T, AccT, false, true, FEW><<<D.max_slots, WG, 0, st>>>(D);
+    else
+        k_g2p<T, AccT, false, false, FEW><<<D.max_slots, WG, 0, st>>>(D);
+}
+
 // The kernels of one substep stage (zmpm_stage_id); launchStep runs all five.
 // more: another substep follows in this call, before anything else.
 template <class T, class AccT>
@@ -634,12 +648,10 @@ void launchStage(zmpm_context* h, int stage, bool more = false)
         }
         break;
     case ZMPM_STAGE_G2P: {
-        if (D.flip)
-            k_g2p<T, AccT, true><<<D.max_slots, WG, 0, st>>>(D);
-        else if (h->variant & VARIANT_G2P_RR)
-            k_g2p<T, AccT, false, true><<<D.max_slots, WG, 0, st>>>(D);
+        if (D.num_mats <= G2P_FEW_MATS)
+            launchG2P<T, AccT, true>(h, D, st);
         else
-            k_g2p<T, AccT, false><<<D.max_slots, WG, 0, st>>>(D);
+            launchG2P<T, AccT, false>(h, D, st);
         // the deferred particles now, or beside the page scan of the call's next
         // substep (the damping passes need them now)
         const int damping = D.flip ? h->desc.pic_damping_iteration : h->desc.rpic_damping_iteration;

@@ -125,6 +125,19 @@ __device__ __forceinline__ const U& uniformAt(const U* table, int i)
     return *(const U*)((Const)reinterpret_cast<uintptr_t>(table) + i);
 }
 
+// f on the record of a lane's scene: with scalar loads where the wavefront's active
+// lanes share it, as nearly all do.  (Vector loads wait for the stores before
+// them, which one counter counts with the loads.)
+template <class T, class AccT, class F>
+__device__ __forceinline__ void withScene(const Dev<T, AccT>& D, int scene, F f)
+{
+    const int first = __builtin_amdgcn_readfirstlane(scene);
+    if (__ballot(scene != first) == 0)
+        f(uniformAt(D.sc, first));
+    else
+        f(D.sc[scene]);
+}
+
 // ---------------------------------------------------------------- positions
 __device__ __forceinline__ int loadPos(const float* base, int i) { return __float_as_int(ldAt(base, i)); }
 __device__ __forceinline__ double loadPos(const double* base, int i) { return ldAt(base, i); }
@@ -329,13 +342,14 @@ __device__ __forceinline__ void binParticle(const Dev<T, AccT>& D, int p, bool a
     uint32_t page = 0xffffffffu - (uint32_t)lane; // inactive lanes never join a run
     int bb[3] = { 0, 0, 0 };
     if (active) {
-        const SceneDev<T>& sd = D.sc[scene];
         int bits = 0;
+        withScene(D, scene, [&](const SceneDev<T>& sd) {
 #pragma unroll
-        for (int a = 0; a < 3; a++) {
-            T d0;
-            bits |= cellOf(x[a], sd.odx, sd.origin[a], sd.domain, bb[a], d0, sd.pos_bits);
-        }
+            for (int a = 0; a < 3; a++) {
+                T d0;
+                bits |= cellOf(x[a], sd.odx, sd.origin[a], sd.domain, bb[a], d0, sd.pos_bits);
+            }
+        });
         if (bits) latch(D.counters, bits);
         uint32_t elem;
         pageElem<T>((uint32_t)bb[0], (uint32_t)bb[1], (uint32_t)bb[2], page, elem);
@@ -2506,10 +2520,16 @@ __device__ __forceinline__ void loadG2PFinish(const Dev<T, AccT>& D, int s, int 
         for (int a = 0; a < 3; a++) r.v[a] = ldAt(P + (PV + a) * cap, p);
 }
 
+// The finish's part of a scene record.
+template <class T>
+struct SceneStep {
+    T dt, dx, odx, Dinv, rpic, pos_scale;
+};
+
 // Returns true for a particle deferred to k_rare (its d, g and stress are
 // completed there).
 template <class T, class AccT, bool FLIP = false>
-__device__ __forceinline__ bool g2pFinish(const Dev<T, AccT>& D, int s, const RawG2P<T>& R, const SceneDev<T>& sd,
+__device__ __forceinline__ bool g2pFinish(const Dev<T, AccT>& D, int s, const RawG2P<T>& R, const SceneStep<T>& sd,
                                           const G2PAcc<T>& A, const MatDev<T>& mt, float* bnd, PosT<T>* xnew)
 {
     bool rare = false;
@@ -2747,16 +2767,27 @@ template <class T, bool FLIP> struct G2PTiles { static constexpr int value = FLI
 
 // RR: workgroups take particle segments round-robin over the XCDs instead of
 // XCD by XCD (an autotuner variant; results are the same).
-template <class T, class AccT, bool FLIP, bool RR = false>
+// FEW: the material table (at most G2P_FEW_MATS, as nearly every program's) is staged
+// in LDS: the finish reads a record many times, between its stores, and each read
+// from memory waits for the stores before it.
+constexpr int G2P_FEW_MATS = 16;
+
+template <class T, class AccT, bool FLIP, bool RR, bool FEW>
 __global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT> D)
 {
     constexpr int NREC = FLIP ? 2 : 1, NT = G2PTiles<T, FLIP>::value;
+    __shared__ MatDev<T> mats[FEW ? G2P_FEW_MATS : 1];
     __shared__ V4<T> gt[NT][NREC][Tile<T>::TN];
     __shared__ int run_block[WG], runs[WG / 64];
     const int lo = (RR ? (int)blockIdx.x : xcdLocal((int)blockIdx.x, (int)gridDim.x)) * WG;
     const int hi = min(lo + WG, D.n);
     const int t = threadIdx.x, s = lo + t;
     const bool live = s < hi;
+    if constexpr (FEW) {
+        static_assert(sizeof(MatDev<T>) % 4 == 0, "material records are copied as words");
+        const int words = min(D.num_mats, G2P_FEW_MATS) * (int)(sizeof(MatDev<T>) / 4);
+        for (int e = t; e < words; e += WG) reinterpret_cast<uint32_t*>(mats)[e] = reinterpret_cast<const uint32_t*>(D.mats)[e];
+    }
     RawG2P<T> R;
     // the Laplacian is gathered for every particle when any material has damage
     // (stored only for damaged ones), so no per-particle material load has to
@@ -2803,7 +2834,11 @@ __global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT>
     float bnd[NSC] = { 0.f, 0.f, 0.f, 0.f, 0.f };
     PosT<T> xnew[3] = { 0, 0, 0 };
     bool rare = false;
-    if (live) rare = g2pFinish<T, AccT, FLIP>(D, s, R, D.sc[scene], A, D.mats[matOf(R.mid)], bnd, xnew);
+    if (live) {
+        SceneStep<T> st;
+        withScene(D, scene, [&](const SceneDev<T>& sd) { st = SceneStep<T> { sd.dt, sd.dx, sd.odx, sd.Dinv, sd.rpic, sd.pos_scale }; });
+        rare = g2pFinish<T, AccT, FLIP>(D, s, R, st, A, FEW ? mats[matOf(R.mid) & (G2P_FEW_MATS - 1)] : D.mats[matOf(R.mid)], bnd, xnew);
+    }
     // deferred particles to the workgroup's rare-path queue, one atomic per wavefront
     const uint64_t rm = __ballot(rare);
     if (rm) {

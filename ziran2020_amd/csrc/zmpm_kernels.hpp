@@ -270,6 +270,7 @@ struct Dev {
     int max_slots;         // workgroups of the particle-order launches (G2P / upload)
     // tables
     const MatDev<T>* mats;
+    int num_mats;
     const ColDev* cols;  // grouped by scene (SceneDev::col0, ncol)
     ColState* colstate;  // [num_cols] states at the running substep's time (written by k_scatter)
     double* bfval;       // [nscenes][MAX_BODY_FORCES][3] body forces at the running substep's time
