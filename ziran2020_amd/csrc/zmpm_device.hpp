@@ -771,12 +771,17 @@ __global__ __launch_bounds__(WG) void k_scatter(Dev<T, AccT> D, int part_wgs, in
 // with their live index (ska / pa); a histogram and cursors group them by cell
 // (skb / pb); then every particle's position is its cell's start plus the
 // number of keys in its cell below its own (all particles ranked in parallel).
-// Blocks larger than the LDS stage take the same steps with the grouped arrays
-// in HBM.  Writes perm, spid, sorted_cell and every cell's start and count, and
+// Blocks larger than the stage group from a second read of HBM into all of the
+// LDS the scatter will use (skm / pm), and blocks larger than that take the same
+// steps with the grouped arrays in HBM.  Writes perm, spid, sorted_cell and every cell's start and count, and
 // leaves the cell counts and starts (relative to the block) in hist / cst.
-template <class T, class AccT>
-__device__ __forceinline__ void blockOrder(const Dev<T, AccT>& D, int b, int start, int cnt, uint32_t* ska, int* pa,
-                                           uint32_t* skb, int* pb, int stage, int* hist, int* cur, int* cst)
+// Of a block that several workgroups share, each orders all and writes its own
+// part [r0, r1) of the positions (all of a block larger than the stage), one of
+// them (cells) the cells' starts and counts.
+template <class T, class AccT, bool PARTS>
+__device__ __forceinline__ void blockOrder(const Dev<T, AccT>& D, int b, int start, int cnt, int r0, int r1, bool cells, uint32_t* ska,
+                                           int* pa, uint32_t* skb, int* pb, int stage, uint32_t* skm, int* pm, int most,
+                                           int* hist, int* cur, int* cst)
 {
     using B = Blk<T>;
     constexpr int bbits = B::xbits + B::ybits + B::zbits;
@@ -821,6 +826,29 @@ __device__ __forceinline__ void blockOrder(const Dev<T, AccT>& D, int b, int sta
         }
     }
     ldsBarrier();
+    // rank inside the cell (keys are unique); write the sorted block.  The cell's
+    // keys are read four at a time so the LDS reads overlap.
+    auto rank = [&](const uint32_t* gk, const int* gp, auto whole) {
+        ldsBarrier();
+        for (int i = t; i < cnt; i += WG) {
+            const uint32_t k = gk[i];
+            const int c = (int)(k >> idbits);
+            const int c0 = cst[c], c1 = c0 + hist[c];
+            if (!whole && (c1 <= r0 || c0 >= r1)) continue;
+            int pos = c0;
+            int j = c0;
+            for (; j + 4 <= c1; j += 4) {
+                const uint32_t k0 = gk[j], k1 = gk[j + 1], k2 = gk[j + 2], k3 = gk[j + 3];
+                pos += (int)(k0 < k) + (int)(k1 < k) + (int)(k2 < k) + (int)(k3 < k);
+            }
+            for (; j < c1; j++) pos += gk[j] < k;
+            if (!whole && (pos < r0 || pos >= r1)) continue;
+            D.perm[start + pos] = gp[i];
+            D.spid[start + pos] = (int)(k & idmask);
+            D.sorted_cell[start + pos] = b * NB + c;
+        }
+    };
+    const bool part = PARTS && r1 - r0 != cnt;
     if (staged) {
         // group by cell
         for (int i = t; i < cnt; i += WG) {
@@ -829,24 +857,35 @@ __device__ __forceinline__ void blockOrder(const Dev<T, AccT>& D, int b, int sta
             skb[dst] = k;
             pb[dst] = pa[i];
         }
-        ldsBarrier();
-        // rank inside the cell (keys are unique); write the sorted block.  The
-        // cell's keys are read four at a time so the LDS reads overlap.
-        for (int i = t; i < cnt; i += WG) {
-            const uint32_t k = skb[i];
-            const int c = (int)(k >> idbits);
-            const int c0 = cst[c], c1 = c0 + hist[c];
-            int pos = c0;
-            int j = c0;
-            for (; j + 4 <= c1; j += 4) {
-                const uint32_t k0 = skb[j], k1 = skb[j + 1], k2 = skb[j + 2], k3 = skb[j + 3];
-                pos += (int)(k0 < k) + (int)(k1 < k) + (int)(k2 < k) + (int)(k3 < k);
+        if (part)
+            rank(skb, pb, std::false_type {});
+        else
+            rank(skb, pb, std::true_type {});
+    }
+    else if (cnt <= most) {
+        for (int i0 = t; i0 < cnt; i0 += 4 * WG) {
+            uint32_t kk[4] = { 0u, 0u, 0u, 0u };
+            int pp[4] = { 0, 0, 0, 0 };
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int i = i0 + u * WG;
+                if (i < cnt) {
+                    kk[u] = D.tmpk[start + i];
+                    pp[u] = D.tmp[start + i];
+                }
             }
-            for (; j < c1; j++) pos += skb[j] < k;
-            D.perm[start + pos] = pb[i];
-            D.spid[start + pos] = (int)(k & idmask);
-            D.sorted_cell[start + pos] = b * NB + c;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if (i0 + u * WG >= cnt) continue;
+                const int dst = atomicAdd(&cur[kk[u] >> idbits], 1);
+                skm[dst] = kk[u];
+                pm[dst] = pp[u];
+            }
         }
+        if (part)
+            rank(skm, pm, std::false_type {});
+        else
+            rank(skm, pm, std::true_type {});
     }
     else {
         // the same in HBM: group into perm/spid, then rank through tmp
@@ -880,7 +919,7 @@ __device__ __forceinline__ void blockOrder(const Dev<T, AccT>& D, int b, int sta
             D.sorted_cell[start + i] = b * NB + c;
         }
     }
-    if (t < NB) {
+    if (cells && t < NB) {
         D.cell_start[b * NB + t] = start + cst[t];
         D.cell_count[b * NB + t] = hist[t];
     }
@@ -1317,32 +1356,62 @@ enum : int { P2G_STD = 0, P2G_MLS = 1, P2G_DAMP = 2 };
 // a result (the in-block order fixes every sum).
 template <class T> struct P2GWaves { static constexpr int value = sizeof(T) == 4 ? 4 : 3; };
 
-template <class T, class AccT, int VAR = P2G_STD, int OCC = P2GWaves<T>::value, bool XCD = false>
-__global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
+// Most workgroups that share a block, and the workgroups (with those of halo
+// blocks, which end at once) up to which blocks are shared.
+constexpr int P2G_MAX_PARTS = 8, P2G_SHARED_WGS = 2048;
+
+// P2G's LDS.
+template <class T, class AccT>
+struct P2GLds {
+    using TL = Tile<T>;
+    V4<T> q[7][TL::CHUNK];
+    T wl[4][TL::CHUNK][3];
+    AccT tile[NGF][TL::TN];
+    int cl[TL::NB], hist[TL::NB], cur[TL::NB], cst[TL::NB], ncl;
+    // cell ranges and neighbours of the block in work and of the one after it
+    struct {
+        int cs[TL::NB], ce[TL::NB], nbl[8];
+    } blk[2];
+    static constexpr int MOST = (int)((sizeof(q) + sizeof(wl) + sizeof(tile)) / 8);
+};
+
+// P2G of the workgroup's blocks.  Where there are workgroups for every block (ONE),
+// each has one: a block, or with several workgroups a block one of its parts
+// (whole chunks, so a lane's partial sums, and with them the FP32 results, are
+// those of an undivided block); each part orders the whole block, and the cell
+// ranges go from the order to the scatter in LDS.  A scene of few blocks otherwise
+// leaves most of the device idle while each block's chunks pass one after the
+// other: event-timed P2G of 512 particles 21.0 -> 13.4 us, of 130,001 (~500 blocks) 40.5 ->
+// 30.3, of 328,509 in 343 blocks 119.5 -> 48.4 (there also by grouping blocks of
+// 1793 particles and more in LDS); with more workgroups than P2G_SHARED_WGS the
+// repeated order and flush cost more than the parts give (262,144 in FP64: 49 us, 68
+// with 4096, 95 with 8192).
+template <class T, class AccT, int VAR, bool ONE>
+__device__ __forceinline__ void p2gBlocks(const Dev<T, AccT>& D, P2GLds<T, AccT>& lds, int nblocks, int wgl, int nwg)
 {
     constexpr bool DAMP = VAR == P2G_DAMP, MLS = VAR == P2G_MLS;
     using B = Blk<T>;
     using TL = Tile<T>;
     constexpr int NB = TL::NB, CH = TL::CHUNK;
     constexpr bool FIXED = std::is_same<AccT, long long>::value;
-    __shared__ V4<T> q[7][CH];
-    __shared__ T wl[4][CH][3];
-    __shared__ AccT tile[NGF][TL::TN];
-    __shared__ int cl[NB];
-    __shared__ int hist[NB], cur[NB], cst[NB];
-    __shared__ int ncl;
-    // cell ranges and neighbours of the block in work and of the one after it
-    __shared__ struct {
-        int cs[NB], ce[NB], nbl[8];
-    } blk[2];
+    auto& q = lds.q;
+    auto& wl = lds.wl;
+    auto& tile = lds.tile;
+    auto& blk = lds.blk;
+    int *const cl = lds.cl, *const hist = lds.hist, *const cur = lds.cur, *const cst = lds.cst;
+    int& ncl = lds.ncl;
     // the in-block sort stages (key, live index) in the payload area and the
-    // grouped copy in the tile area, both free until the block's first chunk
+    // grouped copy in the tile area, both free until the block's first chunk (a
+    // block too large for them is grouped into both areas at once)
     constexpr int SA = (int)(sizeof(q) / 8), SB = (int)(sizeof(tile) / 8);
     constexpr int STAGE = SA < SB ? SA : SB;
     uint32_t* const ska = reinterpret_cast<uint32_t*>(&q[0][0]);
     int* const pa = reinterpret_cast<int*>(&q[0][0]) + SA;
     uint32_t* const skb = reinterpret_cast<uint32_t*>(&tile[0][0]);
     int* const pb = reinterpret_cast<int*>(&tile[0][0]) + SB;
+    constexpr int MOST = P2GLds<T, AccT>::MOST;
+    uint32_t* const skm = reinterpret_cast<uint32_t*>(&lds);
+    int* const pm = reinterpret_cast<int*>(&lds) + MOST;
 
     const int t = threadIdx.x;
     // phase A: particle pt of the chunk.  Float form: two threads per particle,
@@ -1355,33 +1424,41 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     const bool dmg = !DAMP && D.any_damage != 0;
     const int nq = DAMP ? GFO : (dmg ? NGF : GPF);
     const int64_t cap = D.cap, cn = D.cap_nodes;
-    const int nblocks = D.counters[0];
-    // the rare-path queues of this substep's G2P start empty (in k_scatter the
-    // address took its SGPRs past the 96 that 8 wavefronts per SIMD have: 4 % slower)
-    if (!DAMP && blockIdx.x == 0 && t < RARE_QUEUES) D.rare_count[t * RARE_STRIDE] = 0;
-    // and so do the super pages' flags, which every workgroup of the page scan read
-    // (a larger domain's are cleared by k_super_scan)
-    if (!DAMP && D.num_super <= PSCAN_TILE)
-        for (int i = (int)blockIdx.x * WG + t; i < (int)D.num_super; i += (int)gridDim.x * WG) D.super_touched[i] = 0;
+    const int parts = ONE ? max(1, min(P2G_MAX_PARTS, nblocks > 0 ? min(nwg, P2G_SHARED_WGS) / nblocks : 1)) : 1;
+    const int b0 = wgl / parts, part = wgl - parts * b0;
+    if (b0 >= nblocks) return;
+    int r0 = 0, r1 = 0; // ONE: the workgroup's part of its block's particles
+    if constexpr (ONE) {
+        const int cnt = uniformAt(D.block_count, b0), chunks = (cnt + CH - 1) / CH;
+        const int per = (!DAMP && cnt > MOST ? chunks : (chunks + parts - 1) / parts) * CH;
+        r0 = part * per;
+        r1 = min(r0 + per, cnt);
+        if (part > 0 && r0 >= r1) return;
+    }
+    int n0 = 0, n1 = 0;
+    if (ONE && t >= 64) n0 = ldAt(D.nbr, b0 * 8 + (t & 7));
 
     // in-block order of this workgroup's blocks first (a loop of its own, so
     // its registers are free again for the scatter)
-    // blocks round-robin over the XCDs by default: neighbouring blocks flush
-    // their shared halo nodes from different L2s (an XCD-contiguous mapping, as
-    // in G2P, made P2G ~25 % slower on the damage slab); both loops take the
-    // same blocks
-    const int wgl = XCD ? xcdLocal((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
-    for (int b = wgl; !DAMP && b < nblocks; b += gridDim.x) {
+    for (int b = b0; !DAMP && b < nblocks; b += nwg) {
         const int bs = uniformAt(D.block_start, b), cnt = uniformAt(D.block_count, b);
         if (cnt <= 0) { // halo-only block
             if (t < NB) {
                 D.cell_start[b * NB + t] = bs;
                 D.cell_count[b * NB + t] = 0;
             }
+            if (ONE) return;
             continue;
         }
         ldsBarrier(); // LDS of the previous block's order done
-        blockOrder(D, b, bs, cnt, ska, pa, skb, pb, STAGE, hist, cur, cst);
+        blockOrder<T, AccT, ONE>(D, b, bs, cnt, ONE ? r0 : 0, ONE ? r1 : cnt, part == 0, ska, pa, skb, pb, STAGE, skm, pm, MOST, hist, cur, cst);
+        if constexpr (ONE) {
+            if (t < NB) {
+                n0 = bs + cst[t];
+                n1 = hist[t];
+            }
+            break;
+        }
     }
     // the order just written (perm, cell starts) is read below: a full barrier;
     // the loop below exchanges data through LDS only
@@ -1400,9 +1477,9 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     };
     // cell ranges and neighbour table of the workgroup's blocks, loaded two blocks
     // ahead (thread t < NB: start and count of cell t; threads 64..71:
-    // neighbour t - 64), in LDS one block ahead, and combined at their use (summed here, each wait for them
-    // was one for all prefetches, and the sum lived in scratch memory)
-    int n0 = 0, n1 = 0;
+    // neighbour t - 64), in LDS one block ahead, and combined at
+    // their use (summed here, each wait for them was one for all prefetches, and
+    // the sum lived in scratch memory)
     auto fetchBlock = [&](int bb) {
         if (bb >= nblocks) return;
         if (t < 64) {
@@ -1420,21 +1497,26 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
         else if (t >= 64 && t < 72)
             blk[k].nbl[t - 64] = n0;
     };
-    fetchBlock(wgl);
+    if (DAMP || !ONE) fetchBlock(b0);
     keepBlock(0);
-    fetchBlock(wgl + (int)gridDim.x);
+    if (!ONE) fetchBlock(b0 + nwg);
     int par = 0;
-    for (int b = wgl; b < nblocks; b += gridDim.x, par ^= 1) {
+    for (int b = b0; b < nblocks; b += nwg, par ^= 1) {
         ldsBarrier(); // previous block flushed
-        const int bn = b + (int)gridDim.x;
-        keepBlock(par ^ 1);
-        fetchBlock(bn + (int)gridDim.x);
-        ldsBarrier();
+        const int bn = b + nwg;
+        if constexpr (!ONE) {
+            keepBlock(par ^ 1);
+            fetchBlock(bn + nwg);
+            ldsBarrier();
+        }
         const int *const cs = blk[par].cs, *const ce = blk[par].ce, *const nbl = blk[par].nbl;
-        const int bs = cs[0], be = ce[NB - 1];
+        const int bs = ONE ? cs[0] + r0 : cs[0], be = ONE ? cs[0] + r1 : ce[NB - 1];
         // the next block's particles
-        const int ns = blk[par ^ 1].cs[0], ne = bn < nblocks ? blk[par ^ 1].ce[NB - 1] : ns;
-        if (be <= bs) continue; // halo-only block
+        const int ns = ONE ? 0 : blk[par ^ 1].cs[0], ne = !ONE && bn < nblocks ? blk[par ^ 1].ce[NB - 1] : ns;
+        if (be <= bs) { // halo-only block
+            if (ONE) break;
+            continue;
+        }
         for (int e = t; e < nq * TL::TN; e += WG) (&tile[0][0])[e] = AccT(0);
         // the block's scene: its dx and fixed-point scales
         const int bscene = uniformBlockScene(D, b);
@@ -1625,9 +1707,34 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
                     unsafeAtomicAdd(dst, v);
             }
         }
+        if (ONE) break;
     }
     if (ovf & 1) latch(D.counters, ST_OVERFLOW);
     if (ovf & 2) latch(D.counters, ST_CAPACITY);
+}
+
+template <class T, class AccT, int VAR = P2G_STD, int OCC = P2GWaves<T>::value, bool XCD = false>
+__global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
+{
+    __shared__ P2GLds<T, AccT> lds;
+    constexpr bool DAMP = VAR == P2G_DAMP;
+    const int t = threadIdx.x, nwg = (int)gridDim.x, nblocks = D.counters[0];
+    // the rare-path queues of this substep's G2P start empty (in k_scatter the
+    // address took its SGPRs past the 96 that 8 wavefronts per SIMD have: 4 % slower)
+    if (!DAMP && blockIdx.x == 0 && t < RARE_QUEUES) D.rare_count[t * RARE_STRIDE] = 0;
+    // and so do the super pages' flags, which every workgroup of the page scan read
+    // (a larger domain's are cleared by k_super_scan)
+    if (!DAMP && D.num_super <= PSCAN_TILE)
+        for (int i = (int)blockIdx.x * WG + t; i < (int)D.num_super; i += (int)gridDim.x * WG) D.super_touched[i] = 0;
+
+    // blocks round-robin over the XCDs by default: neighbouring blocks flush
+    // their shared halo nodes from different L2s (an XCD-contiguous mapping, as
+    // in G2P, made P2G ~25 % slower on the damage slab)
+    const int wgl = XCD ? xcdLocal((int)blockIdx.x, nwg) : (int)blockIdx.x;
+    if (nblocks <= nwg)
+        p2gBlocks<T, AccT, VAR, true>(D, lds, nblocks, wgl, nwg);
+    else
+        p2gBlocks<T, AccT, VAR, false>(D, lds, nblocks, wgl, nwg);
 }
 
 template <class T, class AccT>
