@@ -308,13 +308,13 @@ zmpm_status allocate(zmpm_context* h, int n)
         ALLOC(D.cgv, 5 * D.cap_nodes);
         ALLOC(D.cgp, 4 * cap);
         ALLOC(D.cg_part, 3 * CG_MAX_WGS);
-        ALLOC(D.cg_bar, 4);
+        ALLOC(D.cg_bar, BAR_STRIDE + BAR_WORDS);
     }
 #undef ALLOC
     if (h->desc.implicit_damage) {
         // k_cg's grid barriers need every workgroup resident: one per CU (the
-        // occupancy calculator must allow at least that; fewer workgroups make
-        // each barrier cheaper, ~9 us at 256)
+        // occupancy calculator must allow at least that; two to a CU change
+        // the solve by 1 %)
         int occ = 0, cus = 0;
         HIPCHK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_cg<T, AccT>, CGW, 0));
         HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->desc.device));
@@ -323,7 +323,7 @@ zmpm_status allocate(zmpm_context* h, int n)
         HIPCHK(h, hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, h->desc.device));
         if (!coop) return fail(h, ZMPM_E_HIP, "the implicit damage solve needs cooperative launches");
         D.cg_wgs = std::max(1, std::min(CG_MAX_WGS, cus));
-        HIPCHK(h, hipMemsetAsync(D.cg_bar, 0, 4 * sizeof(unsigned), h->stream));
+        HIPCHK(h, hipMemsetAsync(D.cg_bar, 0, (BAR_STRIDE + BAR_WORDS) * sizeof(unsigned), h->stream));
     }
     {
         // k_rare walks its queues grid-stride: one resident round of workgroups

@@ -3469,42 +3469,56 @@ constexpr int CG_ITERATIONS = 100;       // ConjugateGradient<..>(100) (AnisoFra
 constexpr double CG_TOLERANCE = 1e-6;    // cg.setTolerance(1e-6) (AnisoFractureSimulation.h:600-601)
 constexpr int CG_SPIN_LIMIT = 1 << 18;   // barrier polls before the wait is given up (ST_BARRIER)
 
-// Barrier over every workgroup of a launch whose workgroups are all resident.
-// arrivals counts up through the launch (cleared before it); barrier number k
-// is passed when it reaches k * nwg.  Release before arriving and acquire after
-// leaving, at agent scope, make each workgroup's writes visible to the others
-// across the chip's L2 slices (one per XCD).  The fences are cache-wide
-// operations, so one wave per workgroup issues them: with every wave fencing,
-// a barrier of 512 workgroups took ~52 us on MI355X, ~22 us with one wave per
-// workgroup, ~9 us with 256 workgroups.  A wait that exceeds the poll limit latches
-// ST_BARRIER and goes on, and once that is latched no barrier waits any more,
-// so the launch always ends soon (with its results flagged as invalid).
-__device__ __forceinline__ void gridBarrier(unsigned* arrivals, unsigned nwg, unsigned& epoch, int* counters)
+// Words that workgroups exchange inside a launch: read and written past the L2s
+// (one per XCD), so a barrier has nothing to write back or to invalidate.
+__device__ __forceinline__ double sharedLoad(const double* p)
 {
-    // every wave's stores complete (in L2) before the workgroup barrier; then
-    // one wave writes the L2 back (agent-scope release) for the whole
-    // workgroup and, after the wait, invalidates it and the CU's vector cache
-    // (agent-scope acquire), which the other waves share
-    __builtin_amdgcn_s_waitcnt(0);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void sharedStore(double* p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Barrier over every workgroup of a launch whose workgroups are all resident.
+// Workgroup w arrives in group w % BAR_GROUPS, the last of a group at the root,
+// and the last of all sets each group's flag to the barrier's number; counters and
+// flags count up through the launch (cleared before it), each in a cache line of its
+// own.  It orders what the workgroups exchange by sharedLoad, sharedStore and
+// device atomics: each is complete before its workgroup arrives.  With ordinary
+// accesses, release and acquire fences at agent scope have to write back and
+// invalidate the L2s (solve of 250,007 particles 136 us instead of 125), and with one
+// counter that all add to and poll the accesses pass one after the other (125 us
+// instead of 106).  A wait that exceeds the poll limit latches ST_BARRIER and
+// goes on, and once that is latched no barrier waits any more, so the launch always
+// ends soon (with its results flagged as invalid).
+__device__ __forceinline__ void gridBarrier(unsigned* bar, unsigned nwg, unsigned& epoch, int* counters)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0); // every access of this wave complete
     __syncthreads();
     epoch++;
     if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const unsigned target = epoch * nwg;
-        unsigned seen = __hip_atomic_fetch_add(arrivals, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        const unsigned g = blockIdx.x % BAR_GROUPS, groups = min(nwg, (unsigned)BAR_GROUPS);
+        const unsigned members = (nwg - g + BAR_GROUPS - 1) / BAR_GROUPS;
+        unsigned* const flag = bar + (1 + BAR_GROUPS + g) * BAR_STRIDE;
+        auto arrive = [](unsigned* at) { return __hip_atomic_fetch_add(at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u; };
+        if (arrive(bar + (1 + g) * BAR_STRIDE) == epoch * members && arrive(bar) == epoch * groups)
+            for (unsigned k = 0; k < groups; k++)
+                __hip_atomic_store(bar + (1 + BAR_GROUPS + k) * BAR_STRIDE, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         int polls = 0;
-        while (seen < target) {
+        while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
             if (++polls > CG_SPIN_LIMIT
-                || (__hip_atomic_load(&counters[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ST_BARRIER)) {
+                || ((polls & 63) == 1
+                    && (__hip_atomic_load(&counters[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ST_BARRIER))) {
                 latch(counters, ST_BARRIER);
                 break;
             }
             __builtin_amdgcn_s_sleep(2);
-            seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
 // Sum over a workgroup of NT threads, the same value in every thread (fixed order).
@@ -3528,7 +3542,7 @@ template <int NT>
 __device__ __forceinline__ double foldPartials(const double* part, int nwg, double* red)
 {
     double v = 0.0;
-    for (int w = threadIdx.x; w < nwg; w += NT) v += part[w];
+    for (int w = threadIdx.x; w < nwg; w += NT) v += sharedLoad(part + w);
     return blockSum<NT>(v, red);
 }
 
@@ -3584,9 +3598,9 @@ __global__ __launch_bounds__(WG) void k_dtilde(Dev<T, AccT> D)
     __shared__ int cs[NB], ce[NB], cl[NB];
     __shared__ int ncl;
     const int t = threadIdx.x;
-    if (blockIdx.x == 0 && t == 0) { // k_cg's barrier arrivals and block tickets
-        D.cg_bar[0] = 0u;
-        D.cg_bar[2] = 0u;
+    if (blockIdx.x == 0) { // k_cg's block tickets and barrier words
+        if (t == 0) D.cg_bar[2] = 0u;
+        for (int k = t; k < BAR_WORDS; k += WG) D.cg_bar[BAR_STRIDE + k] = 0u;
     }
     const int64_t cap = D.cap, cn = D.cap_nodes;
     const int nblocks = D.counters[CNT_BLOCKS];
@@ -3725,10 +3739,10 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
     prr = blockSum<CGW>(prr, red);
     prho = blockSum<CGW>(prho, red);
     if (t == 0) {
-        part[blockIdx.x] = prr;
-        part[CG_MAX_WGS + blockIdx.x] = prho;
+        sharedStore(part + blockIdx.x, prr);
+        sharedStore(part + CG_MAX_WGS + blockIdx.x, prho);
     }
-    gridBarrier(D.cg_bar, (unsigned)nwg, epoch, D.counters);
+    gridBarrier(D.cg_bar + BAR_STRIDE, (unsigned)nwg, epoch, D.counters);
     double rr = foldPartials<CGW>(part, nwg, red);
     double rho = foldPartials<CGW>(part + CG_MAX_WGS, nwg, red);
     const double rel = sqrt(rr) * D.cg_rel;
@@ -3741,12 +3755,12 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
         for (int64_t node = first; node < nn; node += stride) {
             const double dg = DG[node];
             const double mr = dg > 0.0 ? R[node] / dg : 0.0;
-            const double sv = it == 0 ? mr : beta * S[node] + mr;
-            S[node] = sv;
-            Qv[node] = dg * sv;
+            const double sv = it == 0 ? mr : beta * sharedLoad(S + node) + mr;
+            sharedStore(S + node, sv);
+            sharedStore(Qv + node, dg * sv);
             psq += dg * sv * sv;
         }
-        gridBarrier(D.cg_bar, (unsigned)nwg, epoch, D.counters);
+        gridBarrier(D.cg_bar + BAR_STRIDE, (unsigned)nwg, epoch, D.counters);
         // q += K s, one grid block at a time, blocks handed out by a ticket
         // counter (the block sizes vary): s of the block and its halo is staged
         // in LDS; one thread per particle gathers G = sum_j s_j grad w_j and
@@ -3771,7 +3785,7 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
                 if (tb >= 0) {
                     const int elem = ((tx & (TL::BX - 1)) << (B::ybits + B::zbits)) | ((ty & (TL::BY - 1)) << B::zbits)
                         | (tz & (TL::BZ - 1));
-                    v = S[(int64_t)tb * NB + elem];
+                    v = sharedLoad(S + (int64_t)tb * NB + elem);
                 }
                 st[nd] = v;
                 qt[nd] = 0.0;
@@ -3860,8 +3874,8 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
         }
         tickets += (unsigned)(nblocks + nwg);
         psq = blockSum<CGW>(psq, red);
-        if (t == 0) part[2 * CG_MAX_WGS + blockIdx.x] = psq;
-        gridBarrier(D.cg_bar, (unsigned)nwg, epoch, D.counters);
+        if (t == 0) sharedStore(part + 2 * CG_MAX_WGS + blockIdx.x, psq);
+        gridBarrier(D.cg_bar + BAR_STRIDE, (unsigned)nwg, epoch, D.counters);
         const double sq = foldPartials<CGW>(part + 2 * CG_MAX_WGS, nwg, red);
         const double alpha = sq != 0.0 ? rho / sq : 1.7976931348623157e308;
         // x += alpha s, r -= alpha q, and the next M^-1 r . r
@@ -3870,8 +3884,8 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
         for (int64_t node = first; node < nn; node += stride) {
             const double dg = DG[node];
             if (!(dg > 0.0)) continue;
-            X[node] = alpha * S[node] + X[node];
-            const double r = -alpha * Qv[node] + R[node];
+            X[node] = alpha * sharedLoad(S + node) + X[node];
+            const double r = -alpha * sharedLoad(Qv + node) + R[node];
             R[node] = r;
             prr += r * r;
             prho += (r / dg) * r;
@@ -3879,10 +3893,10 @@ __global__ __launch_bounds__(CGW) void k_cg(Dev<T, AccT> D)
         prr = blockSum<CGW>(prr, red);
         prho = blockSum<CGW>(prho, red);
         if (t == 0) {
-            part[blockIdx.x] = prr;
-            part[CG_MAX_WGS + blockIdx.x] = prho;
+            sharedStore(part + blockIdx.x, prr);
+            sharedStore(part + CG_MAX_WGS + blockIdx.x, prho);
         }
-        gridBarrier(D.cg_bar, (unsigned)nwg, epoch, D.counters);
+        gridBarrier(D.cg_bar + BAR_STRIDE, (unsigned)nwg, epoch, D.counters);
         rr = foldPartials<CGW>(part, nwg, red);
         const double rho_new = foldPartials<CGW>(part + CG_MAX_WGS, nwg, red);
         const double conv = sqrt(rr);

@@ -212,6 +212,10 @@ constexpr int RARE_QUEUES = 16, RARE_STRIDE = 32;
 // Entries of a queue: every particle of its workgroups (256 each).
 __host__ __device__ constexpr int64_t rareQueueSize(int wgs) { return (int64_t)((wgs + RARE_QUEUES - 1) / RARE_QUEUES) * 256; }
 
+// The words of k_cg's grid barrier: the root, then a counter and then a flag per
+// group of workgroups, each in a cache line of its own.
+constexpr int BAR_GROUPS = 16, BAR_STRIDE = 32, BAR_WORDS = (1 + 2 * BAR_GROUPS) * BAR_STRIDE;
+
 // Kernel-visible state of one handle.
 template <class T, class AccT>
 struct Dev {
@@ -293,7 +297,7 @@ struct Dev {
     double* cgv;       // [5][cap_nodes] x, r, s, q, diag (x and r first hold sum vol w and the D~ part of rhs)
     T* cgp;            // [4][cap] per sorted particle: d0 x, y, z; vol dt / eta l0^2 (0: not in the solve)
     double* cg_part;   // [3][CG_MAX_WGS] per-workgroup partial sums
-    unsigned* cg_bar;  // [0] barrier arrivals, [1] iterations of the last solve, [2] block tickets
+    unsigned* cg_bar;  // [1] iterations of the last solve, [2] block tickets; from BAR_STRIDE the grid barrier's words
     // scenes
     const SceneDev<T>* sc;     // [nscenes]
     int nscenes;
