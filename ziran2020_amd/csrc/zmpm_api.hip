@@ -134,6 +134,7 @@ struct zmpm_context {
     };
     std::vector<Slot> dl_slots;
     int* dl_bad = nullptr;
+    double* ext_host = nullptr; // pinned rows of zmpm_calculate_dt (16 KiB)
     bool use_graphs = true;
     int fj_state = 0;       // FJMixedMpmForceHelper::state: 0 SOLVE_F, 1 SOLVE_J
     hipError_t launch_err = hipSuccess; // a failed launch that returns its error (the cooperative k_cg)
@@ -1301,6 +1302,7 @@ zmpm_status zmpm_destroy(zmpm_handle h)
         (void)hipEventDestroy(sl.done);
     }
     if (h->dl_bad) (void)hipHostFree(h->dl_bad);
+    if (h->ext_host) (void)hipHostFree(h->ext_host);
     for (void* q : { h->mats_dev, h->cols_dev, h->colstate_dev, h->scenes_dev, h->regions_dev, h->bfval_dev })
         if (q) (void)hipFree(q);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1543,9 +1545,15 @@ static zmpm_status setClocks(zmpm_handle h, const double* dt, const double* t0)
         if (st != ZMPM_OK) return st;
     }
     // each scene's device clock starts at its t0; every substep advances it by its dt
+    double* clock = h->fp32 ? h->Df.clock : h->Dd.clock;
+    if (ns <= CLOCK_ARGS) {
+        ClockArgs a {};
+        std::copy(t0, t0 + ns, a.t0);
+        k_set_clock<<<1, 64, 0, h->stream>>>(clock, a, (int)ns);
+        return ZMPM_OK;
+    }
     h->clock_host.assign(2 * ns, 0.0);
     for (size_t s = 0; s < ns; s++) h->clock_host[2 * s] = h->clock_host[2 * s + 1] = t0[s];
-    double* clock = h->fp32 ? h->Df.clock : h->Dd.clock;
     if (hipMemcpyAsync(clock, h->clock_host.data(), 2 * ns * sizeof(double), hipMemcpyHostToDevice, h->stream) != hipSuccess)
         return fail(h, ZMPM_E_HIP, "clock upload");
     return ZMPM_OK;
@@ -1727,19 +1735,25 @@ zmpm_status zmpm_calculate_dt(zmpm_handle h, double max_dt, double* dt, double* 
     (void)hipSetDevice(h->desc.device);
     double e[8] = { 0, -3.4028234663852886e38, -3.4028234663852886e38, -3.4028234663852886e38,
                     -3.4028234663852886e38, -3.4028234663852886e38, -3.4028234663852886e38, 0 };
-    double* ext = h->fp32 ? h->Df.extent : h->Dd.extent;
-    if (h->n > 0 && ext) {
+    if (h->n > 0 && (h->fp32 ? h->Df.extent : h->Dd.extent)) {
+        // the workgroups' maxima straight into pinned memory, folded here: one launch
+        // and no copy (a second launch and a copy were 20 us of a small scene's step)
+        if (!h->ext_host) HIPCHK(h, hipHostMalloc((void**)&h->ext_host, EXTENT_WGS * 8 * sizeof(double)));
+        const int rows = gridFor(h->n, WG, EXTENT_WGS);
         if (h->fp32) {
-            k_extent<float, long long><<<EXTENT_WGS, WG, 0, h->stream>>>(h->Df, 0, EXTENT_WGS, nullptr, 0.0, 0.0);
-            k_extent<float, long long><<<1, WG, 0, h->stream>>>(h->Df, 1, EXTENT_WGS, nullptr, 0.0, 0.0);
+            Dev<float, long long> D = h->Df;
+            D.extent = h->ext_host;
+            k_extent<float, long long><<<rows, WG, 0, h->stream>>>(D, 0, rows, nullptr, 0.0, 0.0);
         }
         else {
-            k_extent<double, double><<<EXTENT_WGS, WG, 0, h->stream>>>(h->Dd, 0, EXTENT_WGS, nullptr, 0.0, 0.0);
-            k_extent<double, double><<<1, WG, 0, h->stream>>>(h->Dd, 1, EXTENT_WGS, nullptr, 0.0, 0.0);
+            Dev<double, double> D = h->Dd;
+            D.extent = h->ext_host;
+            k_extent<double, double><<<rows, WG, 0, h->stream>>>(D, 0, rows, nullptr, 0.0, 0.0);
         }
         HIPCHK(h, hipGetLastError());
-        HIPCHK(h, hipMemcpyAsync(e, ext + EXTENT_WGS * 8, 8 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
+        for (int r = 0; r < rows; r++)
+            for (int k = 0; k < 8; k++) e[k] = std::fmax(e[k], h->ext_host[8 * r + k]);
     }
     if (max_speed) *max_speed = e[0];
     for (int a = 0; a < 3; a++) {
