@@ -260,11 +260,21 @@ __device__ __forceinline__ void pageElem(uint32_t i, uint32_t j, uint32_t k, uin
 }
 
 // ---------------------------------------------------------------- wave scans
+// The wavefront's maximum in every lane, all lanes active: along rows of 16, then
+// row to row, by data-parallel moves in the vector unit (shuffles pass through LDS,
+// one after the other).
 __device__ __forceinline__ float waveMax(float v)
 {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
-    return v;
+#define ZMPM_DPP_MAX(ctrl, rows)                                                                                        \
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xf, false)))
+    ZMPM_DPP_MAX(0x111, 0xf); // from 1, 2, 4 and 8 lanes below in the row
+    ZMPM_DPP_MAX(0x112, 0xf);
+    ZMPM_DPP_MAX(0x114, 0xf);
+    ZMPM_DPP_MAX(0x118, 0xf);
+    ZMPM_DPP_MAX(0x142, 0xa); // rows 1 and 3 from the row below
+    ZMPM_DPP_MAX(0x143, 0xc); // rows 2 and 3 from row 1
+#undef ZMPM_DPP_MAX
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 __device__ __forceinline__ int waveInclusiveScan(int v)
@@ -366,6 +376,7 @@ __device__ __forceinline__ void binParticle(const Dev<T, AccT>& D, int p, bool a
     if (active && head) {
         slot = atomicAdd(&D.page_count[page], next - lane);
         const uint32_t Bx = bb[0] >> B::xbits, By = bb[1] >> B::ybits, Bz = bb[2] >> B::zbits;
+        uint32_t super = 0xffffffffu;
 #pragma unroll
         for (int a = 0; a < 2; a++)
 #pragma unroll
@@ -374,7 +385,9 @@ __device__ __forceinline__ void binParticle(const Dev<T, AccT>& D, int p, bool a
                 for (int c = 0; c < 2; c++) {
                     const uint32_t pg = pageOfBlock<T>(D.masks, Bx + a, By + b, Bz + c);
                     D.touched[pg] = 1;
-                    D.super_touched[pg / PSCAN_TILE] = 1;
+                    // (neighbours are mostly in one super page, whose flag is one word for
+                    // hundreds of wavefronts)
+                    if (pg / PSCAN_TILE != super) D.super_touched[super = pg / PSCAN_TILE] = 1;
                 }
     }
     slot = __shfl(slot, start);
