@@ -1945,7 +1945,7 @@ done:
 
 // Key of the tuning cache: the device and what selects the work and the kernels.
 // Raised when the kernels change enough that cached tunings should be redone.
-constexpr int kTuneRevision = 4;
+constexpr int kTuneRevision = 5;
 
 static std::string tuneKey(zmpm_handle h, int32_t tune_variants)
 {
