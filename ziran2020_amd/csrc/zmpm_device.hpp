@@ -1408,7 +1408,7 @@ struct P2GLds {
 // ranges go from the order to the scatter in LDS.  A scene of few blocks otherwise
 // leaves most of the device idle while each block's chunks pass one after the
 // other: event-timed P2G of 512 particles 21.0 -> 13.4 us, of 130,001 (~500 blocks) 40.5 ->
-// 30.3, of 328,509 in 343 blocks 119.5 -> 48.4 (there also by grouping blocks of
+// 28.8, of 328,509 in 343 blocks 119.5 -> 43.2 (there also by grouping blocks of
 // 1793 particles and more in LDS); with more workgroups than P2G_SHARED_WGS the
 // repeated order and flush cost more than the parts give (262,144 in FP64: 49 us, 68
 // with 4096, 95 with 8192).
@@ -1450,9 +1450,13 @@ __device__ __forceinline__ void p2gBlocks(const Dev<T, AccT>& D, P2GLds<T, AccT>
     const bool dmg = !DAMP && D.any_damage != 0;
     const int nq = DAMP ? GFO : (dmg ? NGF : GPF);
     const int64_t cap = D.cap, cn = D.cap_nodes;
-    const int parts = ONE ? max(1, min(P2G_MAX_PARTS, nblocks > 0 ? min(nwg, P2G_SHARED_WGS) / nblocks : 1)) : 1;
-    const int b0 = wgl / parts, part = wgl - parts * b0;
-    if (b0 >= nblocks) return;
+    const int parts = ONE ? max(1, min(P2G_MAX_PARTS, min(nwg, P2G_SHARED_WGS) / nblocks)) : 1;
+    // every block's first part, then the second ones: the workgroups with work are
+    // the first of the grid and so spread over the XCDs, whatever the number of parts
+    // (a block's parts side by side: P2G of 250,007 particles in ~790 blocks 43.5 us
+    // instead of 36.7, of 328,509 in 343 blocks 47.9 instead of 43.2)
+    const int part = ONE ? wgl / nblocks : 0, b0 = wgl - part * nblocks;
+    if (ONE ? part >= parts : b0 >= nblocks) return;
     int r0 = 0, r1 = 0; // ONE: the workgroup's part of its block's particles
     if constexpr (ONE) {
         const int cnt = uniformAt(D.block_count, b0), chunks = (cnt + CH - 1) / CH;
@@ -1757,6 +1761,7 @@ __global__ __launch_bounds__(WG, OCC) void k_p2g(Dev<T, AccT> D)
     // their shared halo nodes from different L2s (an XCD-contiguous mapping, as
     // in G2P, made P2G ~25 % slower on the damage slab)
     const int wgl = XCD ? xcdLocal((int)blockIdx.x, nwg) : (int)blockIdx.x;
+    if (nblocks == 0) return;
     if (nblocks <= nwg)
         p2gBlocks<T, AccT, VAR, true>(D, lds, nblocks, wgl, nwg);
     else
