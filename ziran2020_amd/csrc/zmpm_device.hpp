@@ -83,9 +83,10 @@ __device__ __forceinline__ int xcdLocal(int wg, int nwg)
 
 // ------------------------------------------------------- particle field access
 // Element i of a field whose base (buffer + field * capacity) is uniform: the
-// byte offset is formed in 32 bits (capacity < 2^27), so the access takes the
-// scalar-base + 32-bit vector-offset addressing form and needs no per-lane
-// 64-bit address arithmetic.
+// byte offset is formed in 32 bits (capacity < 2^27; a table with entries per
+// cell goes through its block's row, blockRow), so the access takes the
+// scalar-base + 32-bit vector-offset addressing form and needs no per-lane 64-bit
+// address arithmetic.
 // The base goes through readfirstlane (a no-op on a uniform value) so the
 // optimiser keeps it a scalar instead of folding the field offset into the
 // per-lane address; the access stays in the global address space.
@@ -1509,15 +1510,18 @@ __device__ __forceinline__ void p2gBlocks(const Dev<T, AccT>& D, P2GLds<T, AccT>
     // ahead (thread t < NB: start and count of cell t; threads 64..71:
     // neighbour t - 64), in LDS one block ahead, and combined at
     // their use (summed here, each wait for them was one for all prefetches, and
-    // the sum lived in scratch memory)
+    // the sum lived in scratch memory).  Rows are those of the even block below, so
+    // a lane's index changes with the block: fixed indices stay in registers (24 B
+    // of scratch in the double form instead of 12, 12 in the float form instead of 0)
     auto fetchBlock = [&](int bb) {
         if (bb >= nblocks) return;
+        const int half = bb & 1, row = bb - half;
         if (t < 64) {
-            n0 = ldAt(D.cell_start, bb * NB + (t & (NB - 1)));
-            n1 = ldAt(D.cell_count, bb * NB + (t & (NB - 1)));
+            n0 = ldAt(blockRow<NB>(D.cell_start, row), half * NB + (t & (NB - 1)));
+            n1 = ldAt(blockRow<NB>(D.cell_count, row), half * NB + (t & (NB - 1)));
         }
         else
-            n0 = ldAt(D.nbr, bb * 8 + (t & 7));
+            n0 = ldAt(blockRow<8>(D.nbr, row), half * 8 + (t & 7));
     };
     auto keepBlock = [&](int k) {
         if (t < NB) {

@@ -216,6 +216,15 @@ __host__ __device__ constexpr int64_t rareQueueSize(int wgs) { return (int64_t)(
 // group of workgroups, each in a cache line of its own.
 constexpr int BAR_GROUPS = 16, BAR_STRIDE = 32, BAR_WORDS = (1 + 2 * BAR_GROUPS) * BAR_STRIDE;
 
+// Row of block b in a table with ROW entries per block.  Formed in 64 bits: such
+// tables may have 2^31 entries, more than a byte offset of 32 bits reaches from
+// their start (cell_start's would wrap from block 2^24 on in the float form).
+template <int ROW, class U>
+__host__ __device__ constexpr U* blockRow(U* table, int b)
+{
+    return table + (int64_t)b * ROW;
+}
+
 // Kernel-visible state of one handle.
 template <class T, class AccT>
 struct Dev {
