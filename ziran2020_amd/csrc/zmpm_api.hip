@@ -894,6 +894,7 @@ zmpm_status downloadT(zmpm_context* h, zmpm_particles* p)
     if (st != ZMPM_OK) return st;
     *h->dl_bad = 0;
     k_export_index<T, AccT><<<gridFor(n, WG, 1 << 30), WG, 0, h->stream>>>(D, h->dl_bad);
+    HIPCHK(h, hipGetLastError()); // kept per host thread: the others would not see it
     std::atomic<int64_t> next { 0 };
     std::atomic<int> error { (int)hipSuccess };
     auto participate = [&](int slot) {
