@@ -13,6 +13,7 @@
 #include <sstream>
 #include <limits>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -828,28 +829,92 @@ zmpm_status restress(zmpm_context* h)
 constexpr size_t kSlotBytes = 4u << 20;
 constexpr int kMaxSlots = 8;
 
+// Pinned host memory, or null.
+void* pinned(size_t bytes)
+{
+    void* p = nullptr;
+    if (hipHostMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // The handle's pinned buffers for `want` participants and `bytes` in all (kept
 // until the handle ends, 32 MiB at most; a buffer grows to what is asked of it).
-zmpm_status downloadSlots(zmpm_context* h, int want, size_t bytes)
+// Returns for how many participants there is memory.
+int downloadSlots(zmpm_context* h, int want, size_t bytes)
 {
-    if (!h->dl_bad) HIPCHK(h, hipHostMalloc((void**)&h->dl_bad, sizeof(int)));
-    while ((int)h->dl_slots.size() < want) {
-        zmpm_context::Slot sl;
-        HIPCHK(h, hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
-        h->dl_slots.push_back(sl);
-    }
+    const size_t need = std::min(kSlotBytes, std::max<size_t>(bytes, 4096));
+    if (!h->dl_bad) h->dl_bad = static_cast<int*>(pinned(sizeof(int)));
+    if (!h->dl_bad) return 0;
     for (int k = 0; k < want; k++) {
+        if (k == (int)h->dl_slots.size()) {
+            zmpm_context::Slot sl;
+            if (hipEventCreateWithFlags(&sl.done, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return k;
+            }
+            h->dl_slots.push_back(sl);
+        }
         zmpm_context::Slot& sl = h->dl_slots[(size_t)k];
-        const size_t need = std::min(kSlotBytes, std::max<size_t>(bytes, 4096));
         if (sl.size >= need) continue;
         if (sl.host) (void)hipHostFree(sl.host);
-        sl.host = nullptr;
-        sl.size = 0;
-        if (hipHostMalloc(&sl.host, need) != hipSuccess) {
-            (void)hipGetLastError();
-            return fail(h, ZMPM_E_NOMEM, "no pinned memory for the download");
+        sl.host = pinned(need);
+        sl.size = sl.host ? need : 0;
+        if (!sl.host) return k;
+    }
+    return want;
+}
+
+// The requested arrays one behind the other, and where each goes.
+struct Download {
+    ExportJobs J {};
+    char* dst[EXP_MAX];
+    size_t row_bytes[EXP_MAX];
+};
+
+// Without pinned memory: the fields as stored, and their rows put into the
+// caller's order here.
+template <class T, class AccT>
+zmpm_status downloadPageable(zmpm_context* h, const Download& L)
+{
+    const Dev<T, AccT>& D = devOf<T, AccT>(h);
+    constexpr bool F32 = std::is_same<T, float>::value;
+    const size_t n = (size_t)h->n;
+    std::vector<int> ids(n), mat(n);
+    std::vector<T> col(n);
+    HIPCHK(h, hipMemcpyAsync(ids.data(), D.pid, n * sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipMemcpyAsync(mat.data(), D.pmat, n * sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    for (size_t s = 0; s < n; s++)
+        if ((size_t)(unsigned)ids[s] >= n || (size_t)(unsigned)(mat[s] >> PMAT_SCENE_SHIFT) >= h->scenes.size())
+            return fail(h, ZMPM_E_HIP, "corrupt particle id or scene table");
+    for (int j = 0; j < L.J.count; j++) {
+        const int width = L.J.width[j], kind = L.J.kind[j];
+        double* const out = reinterpret_cast<double*>(L.dst[j]);
+        if (kind == EXP_MAT || kind == EXP_ZERO) {
+            for (size_t s = 0; s < n; s++)
+                if (kind == EXP_MAT)
+                    reinterpret_cast<int32_t*>(L.dst[j])[ids[s]] = mat[s] & PMAT_MAT_MASK;
+                else
+                    out[s] = 0.0;
+            continue;
         }
-        sl.size = need;
+        for (int k = 0; k < width; k++) {
+            HIPCHK(h, hipMemcpyAsync(col.data(), D.P + (L.J.field[j] + k) * D.cap, n * sizeof(T), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(h, hipStreamSynchronize(h->stream));
+            const double add = F32 && (kind == EXP_J || (kind == EXP_F && k % 4 == 0)) ? 1.0 : 0.0;
+            for (size_t s = 0; s < n; s++) {
+                double v = (double)col[s];
+                if (F32 && kind == EXP_POS) {
+                    int X;
+                    std::memcpy(&X, &col[s], sizeof(int));
+                    const zmpm_scene_desc& sd = h->scenes[(size_t)(mat[s] >> PMAT_SCENE_SHIFT)];
+                    v = X == POS_NAN ? std::numeric_limits<double>::quiet_NaN()
+                                     : (double)X * sd.dx / (double)(1 << posBits(sd.domain_nodes));
+                }
+                out[(size_t)ids[s] * width + k] = add != 0.0 ? v + add : v;
+            }
+        }
     }
     return ZMPM_OK;
 }
@@ -860,17 +925,16 @@ zmpm_status downloadT(zmpm_context* h, zmpm_particles* p)
     const Dev<T, AccT>& D = devOf<T, AccT>(h);
     const int64_t n = h->n;
     if (n == 0) return ZMPM_OK;
-    ExportJobs J {};
-    char* dst[EXP_MAX];
-    size_t row_bytes[EXP_MAX];
+    Download L;
+    ExportJobs& J = L.J;
     auto add = [&](void* to, int field, int width, int kind) {
         if (!to) return;
         const int j = J.count++;
-        dst[j] = static_cast<char*>(to);
+        L.dst[j] = static_cast<char*>(to);
         J.field[j] = field;
         J.width[j] = width;
         J.kind[j] = kind;
-        row_bytes[j] = kind == EXP_MAT ? sizeof(int32_t) : (size_t)width * sizeof(double);
+        L.row_bytes[j] = kind == EXP_MAT ? sizeof(int32_t) : (size_t)width * sizeof(double);
         J.off[j + 1] = J.off[j] + (kind == EXP_MAT ? (n + 1) / 2 : n * width);
     };
     add(p->x, PX, 3, EXP_POS);
@@ -889,9 +953,17 @@ zmpm_status downloadT(zmpm_context* h, zmpm_particles* p)
     const int64_t words = J.off[J.count];
     const int64_t chunk = (int64_t)(kSlotBytes / sizeof(double));
     const int64_t nchunks = (words + chunk - 1) / chunk;
-    const int want = (int)std::min<int64_t>(nchunks, std::min(kMaxSlots, std::max(1, (int)std::thread::hardware_concurrency())));
-    zmpm_status st = downloadSlots(h, std::max(want, 1), (size_t)words * sizeof(double));
-    if (st != ZMPM_OK) return st;
+    const int threads_here = std::max(1, (int)std::thread::hardware_concurrency());
+    const int most = (int)std::min<int64_t>(std::max<int64_t>(nchunks, 1), std::min(kMaxSlots, threads_here));
+    const int want = downloadSlots(h, most, (size_t)words * sizeof(double));
+    if (want == 0) {
+        try {
+            return downloadPageable<T, AccT>(h, L);
+        }
+        catch (const std::bad_alloc&) {
+            return fail(h, ZMPM_E_NOMEM, "no host memory for the download");
+        }
+    }
     *h->dl_bad = 0;
     k_export_index<T, AccT><<<gridFor(n, WG, 1 << 30), WG, 0, h->stream>>>(D, h->dl_bad);
     HIPCHK(h, hipGetLastError()); // kept per host thread: the others would not see it
@@ -915,8 +987,8 @@ zmpm_status downloadT(zmpm_context* h, zmpm_particles* p)
                 const int64_t a = std::max(w0, J.off[j]), b = std::min(w1, J.off[j + 1]);
                 if (a >= b) continue;
                 const size_t at = (size_t)(a - J.off[j]) * sizeof(double);
-                const size_t len = std::min((size_t)(b - a) * sizeof(double), (size_t)n * row_bytes[j] - at);
-                std::memcpy(dst[j] + at, static_cast<const char*>(sl.host) + (size_t)(a - w0) * sizeof(double), len);
+                const size_t len = std::min((size_t)(b - a) * sizeof(double), (size_t)n * L.row_bytes[j] - at);
+                std::memcpy(L.dst[j] + at, static_cast<const char*>(sl.host) + (size_t)(a - w0) * sizeof(double), len);
             }
         }
     };
