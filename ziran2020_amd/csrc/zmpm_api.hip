@@ -305,7 +305,7 @@ zmpm_status allocate(zmpm_context* h, int n)
     ALLOC(D.oldv, 4 * D.cap_nodes);
     ALLOC(D.scales, NSC * ns);
     ALLOC(D.maxbits, (int64_t)NSC * BOUND_SLOTS * ns);
-    ALLOC(D.extent, (int64_t)(EXTENT_WGS + 1) * 8);
+    ALLOC(D.extent, (int64_t)EXTENT_WGS * 8);
     if (h->desc.implicit_damage) {
         ALLOC(D.cgv, 5 * D.cap_nodes);
         ALLOC(D.cgp, 4 * cap);
@@ -1808,25 +1808,31 @@ zmpm_status zmpm_calculate_dt(zmpm_handle h, double max_dt, double* dt, double* 
     (void)hipSetDevice(h->desc.device);
     double e[8] = { 0, -3.4028234663852886e38, -3.4028234663852886e38, -3.4028234663852886e38,
                     -3.4028234663852886e38, -3.4028234663852886e38, -3.4028234663852886e38, 0 };
-    if (h->n > 0 && (h->fp32 ? h->Df.extent : h->Dd.extent)) {
+    if (h->n > 0) {
         // the workgroups' maxima straight into pinned memory, folded here: one launch
-        // and no copy (a second launch and a copy were 20 us of a small scene's step)
-        if (!h->ext_host) HIPCHK(h, hipHostMalloc((void**)&h->ext_host, EXTENT_WGS * 8 * sizeof(double)));
+        // and no copy (a second launch and a copy were 20 us of a small scene's step);
+        // without pinned memory through the handle's device rows
+        if (!h->ext_host) h->ext_host = static_cast<double*>(pinned(EXTENT_WGS * 8 * sizeof(double)));
         const int rows = gridFor(h->n, WG, EXTENT_WGS);
         if (h->fp32) {
             Dev<float, long long> D = h->Df;
-            D.extent = h->ext_host;
+            if (h->ext_host) D.extent = h->ext_host;
             k_extent<float, long long><<<rows, WG, 0, h->stream>>>(D, 0, rows, nullptr, 0.0, 0.0);
         }
         else {
             Dev<double, double> D = h->Dd;
-            D.extent = h->ext_host;
+            if (h->ext_host) D.extent = h->ext_host;
             k_extent<double, double><<<rows, WG, 0, h->stream>>>(D, 0, rows, nullptr, 0.0, 0.0);
         }
         HIPCHK(h, hipGetLastError());
+        double copied[EXTENT_WGS * 8];
+        if (!h->ext_host)
+            HIPCHK(h, hipMemcpyAsync(copied, h->fp32 ? h->Df.extent : h->Dd.extent, (size_t)rows * 8 * sizeof(double),
+                                     hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
-        for (int r = 0; r < rows; r++)
-            for (int k = 0; k < 8; k++) e[k] = std::fmax(e[k], h->ext_host[8 * r + k]);
+        const double* row = h->ext_host ? h->ext_host : copied;
+        for (int r = 0; r < rows; r++, row += 8)
+            for (int k = 0; k < 8; k++) e[k] = std::fmax(e[k], row[k]);
     }
     if (max_speed) *max_speed = e[0];
     for (int a = 0; a < 3; a++) {

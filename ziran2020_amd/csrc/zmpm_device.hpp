@@ -3328,9 +3328,10 @@ __global__ __launch_bounds__(WG) void k_damp_g2p(Dev<T, AccT> D)
 
 // evalMaxParticleSpeed (MpmSimulationBase.cpp:1613-1638): per workgroup the
 // maxima of |v| (in the particle precision, as the reference's velocity.norm()),
-// x and -x over a grid stride of the particles; the last launch folds the
-// EXTENT_WGS partials into row EXTENT_WGS.  Empty: speed 0, corners at the
-// reference's initial float lowest.
+// x and -x over a grid stride of the particles, a row of 8 each; zmpm_calculate_dt
+// folds the rows on the host, zmpm_calculate_dt_noalloc by a second launch (fold)
+// into the row after them.  Empty: speed 0, corners at the reference's initial
+// float lowest.
 constexpr int EXTENT_WGS = 256;
 
 __device__ __forceinline__ double posMetres(int X, double dx, int pb) { return (double)X * dx * (1.0 / (double)(1 << pb)); }
