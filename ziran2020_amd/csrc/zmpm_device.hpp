@@ -691,19 +691,6 @@ __device__ __forceinline__ float boundScale(float m, float fallback)
     return ldexpf(1.0f, se);
 }
 
-// The start times of a run's scenes, few enough to travel as a kernel's argument (a
-// copy from host memory costs a step of a small scene several times this launch).
-constexpr int CLOCK_ARGS = 16;
-struct ClockArgs {
-    double t0[CLOCK_ARGS];
-};
-
-__global__ __launch_bounds__(64) void k_set_clock(double* clock, ClockArgs a, int nscenes)
-{
-    const int s = threadIdx.x;
-    if (s < nscenes && s < CLOCK_ARGS) clock[2 * s] = clock[2 * s + 1] = a.t0[s];
-}
-
 template <class T, class AccT>
 __device__ __forceinline__ void beginStep(const Dev<T, AccT>& D)
 {
