@@ -39,3 +39,31 @@ def test_parts(gpu, oracle, precision, transfer, n):
         assert normwise(out[0][k], out[2][k]) < TOL[precision], k
         assert normwise(out[1][k], out[2][k]) < TOL[precision], k
         assert precision == A.PREC_FP64 or np.array_equal(out[0][k], out[1][k]), k
+
+
+def grid_blocks(sc):
+    """The float form's 4x4x4-node blocks that the particles' stencils may reach."""
+    b = np.unique(np.floor(sc.x / sc.dx - 0.5).astype(int) // 4, axis=0)
+    halo = np.stack(np.meshgrid(*[(0, 1)] * 3, indexing="ij"), -1).reshape(-1, 1, 3)
+    return len(np.unique((b + halo).reshape(-1, 3), axis=0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", range(16))
+@pytest.mark.parametrize("share", (8, 2, 1))
+def test_parts_in_every_variant(gpu, variant, share):
+    """Every compiled variant where each block has workgroups of its own: eight (the default), two and one,
+    with some left over and in no multiple of the XCDs."""
+    sc = scenes.damage_slab(n=8000, dx=1 / 64, size=(0.5, 0.15, 0.15), domain_nodes=128, sigma_crit=20.0, pull_speed=0.5)
+    blocks = grid_blocks(sc)
+    assert 200 < blocks < 2048 // 8
+    one, sim = sc.make(gpu, A.PREC_FP32), sc.make(gpu, A.PREC_FP32)
+    one.set_launch_config(p2g_wgs=1, variant=0)
+    sim.set_launch_config(variant=variant, **({} if share == 8 else dict(p2g_wgs=share * blocks + blocks // 4 | 1)))
+    out = []
+    for s in (one, sim):
+        sc.run(s, 4)
+        out.append(s.download())
+    for k in ("x", "v", "C", "F", "d", "g"):
+        assert np.array_equal(out[0][k], out[1][k]), k
+    assert out[0]["d"].max() > 0
