@@ -40,7 +40,7 @@ typedef enum {
     ZMPM_E_CFL = 4,      /* a particle moved more than dx in one substep          */
     ZMPM_E_NAN = 5,      /* non-finite particle position                          */
     ZMPM_E_OVERFLOW = 6, /* 64-bit fixed-point P2G accumulator out of range       */
-    ZMPM_E_NOMEM = 7     /* device allocation failed                              */
+    ZMPM_E_NOMEM = 7     /* device (download: host) allocation failed             */
 } zmpm_status;
 
 /* Precision form chosen at create time. */
@@ -298,7 +298,10 @@ zmpm_status zmpm_clear_colliders(zmpm_handle h);
 /* Particle state in / out.  Upload replaces the scene-building writes of
  * MpmInitializationHelper::sampleInAnalyticLevelSet (MpmInitializationHelper.h:637-647);
  * download returns particles in their upload order (the reference never
- * reorders the DataManager arrays). */
+ * reorders the DataManager arrays).  It copies with up to eight host threads, which
+ * end before it returns, through pinned buffers that the first download allocates
+ * and the handle keeps (32 MiB at most; with less pinned memory it uses fewer, and
+ * with none pageable memory). */
 zmpm_status zmpm_upload(zmpm_handle h, const zmpm_particles* p);
 zmpm_status zmpm_download(zmpm_handle h, zmpm_particles* p);
 
@@ -431,7 +434,8 @@ zmpm_status zmpm_get_timings(zmpm_handle h, int32_t* count, const char** names, 
  * max speed, or max_dt when every particle is at rest (collision-object speeds
  * are not included, as in the reference); for a batch the smallest of the
  * scenes' steps and the box over the scenes' own frames.  Output pointers may
- * be NULL; min_corner / max_corner take 3 doubles. */
+ * be NULL; min_corner / max_corner take 3 doubles.  The first call allocates 16 KiB
+ * of pinned memory, which the handle keeps (without it, device rows are copied). */
 zmpm_status zmpm_calculate_dt(zmpm_handle h, double max_dt, double* dt, double* max_speed, double* min_corner,
                               double* max_corner);
 

@@ -825,7 +825,11 @@ zmpm_status restress(zmpm_context* h)
 // Downloads go through pinned buffers of at most kSlotBytes, one per
 // participating host thread: each thread takes the next range of words, has
 // k_export write it into its buffer and copies it on to the caller's arrays, so
-// the transfer of one range runs beside the host copies of the others.
+// the transfer of one range runs beside the host copies of the others.  Download
+// of 10.4M particles' x, v, C, F and d: 41.0 ms, the first one into new arrays 45 to 47
+// (four buffers: 40.9, but 57 the first time; 16: 41.0 and 43); with 1 MiB buffers
+// 48.7, with 16 MiB ones 40.2, but the first download of 1M particles, which
+// allocates them, 14 ms instead of 8.5.
 constexpr size_t kSlotBytes = 4u << 20;
 constexpr int kMaxSlots = 8;
 

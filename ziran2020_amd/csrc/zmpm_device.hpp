@@ -4,9 +4,11 @@
 // One substep (Ziran MpmSimulationBase::advanceOneTimeStep,
 // Lib/MPM/MpmSimulationBase.cpp:262-357) is this launch sequence on the
 // handle's stream:
-//   k_super_scan     touched super pages in order (single-pass compaction)
+//   k_super_scan     (domains of more than 2048 super pages only) touched super
+//                    pages in order (single-pass compaction)
 //   k_page_scan      dense block ids in page (Morton) order, page table, block
-//                    ranges (single-pass scan)
+//                    ranges (single-pass scan); from a call's second substep on
+//                    k_page_scan_rare, with k_rare's work of the substep before
 //   k_scatter        particles to their block ranges; zero block accumulators,
 //                    forward-neighbour block table, device clock and
 //                    fixed-point scales (float form)
@@ -26,7 +28,9 @@
 //                    and bins them for the next substep (binParticle: key,
 //                    page activation, per-page counts)
 //   k_rare           the particles k_g2p deferred (full damage update,
-//                    near-inversion stress, plasticity return mappings)
+//                    near-inversion stress, plasticity return mappings): after
+//                    a call's last substep, and before damping passes
+// Downloads are k_export_index and k_export, the CFL step is k_extent.
 #pragma once
 #include "zmpm_kernels.hpp"
 
@@ -1395,9 +1399,9 @@ struct P2GLds {
 // those of an undivided block); each part orders the whole block, and the cell
 // ranges go from the order to the scatter in LDS.  A scene of few blocks otherwise
 // leaves most of the device idle while each block's chunks pass one after the
-// other: event-timed P2G of 512 particles 21.0 -> 13.4 us, of 130,001 (~500 blocks) 40.5 ->
-// 28.8, of 328,509 in 343 blocks 119.5 -> 43.2 (there also by grouping blocks of
-// 1793 particles and more in LDS); with more workgroups than P2G_SHARED_WGS the
+// other: event-timed P2G of 512 particles 21.0 -> 13.9 us, of 130,001 (681 blocks,
+// 447 of them with particles) 40.5 -> 28.8, of 328,509 (512, 343) 119.5 -> 43.5 (there
+// also by grouping blocks of 1793 particles and more in LDS); with more workgroups than P2G_SHARED_WGS the
 // repeated order and flush cost more than the parts give (262,144 in FP64: 49 us, 68
 // with 4096, 95 with 8192).
 template <class T, class AccT, int VAR, bool ONE>
@@ -1441,8 +1445,9 @@ __device__ __forceinline__ void p2gBlocks(const Dev<T, AccT>& D, P2GLds<T, AccT>
     const int parts = ONE ? max(1, min(P2G_MAX_PARTS, min(nwg, P2G_SHARED_WGS) / nblocks)) : 1;
     // every block's first part, then the second ones: the workgroups with work are
     // the first of the grid and so spread over the XCDs, whatever the number of parts
-    // (a block's parts side by side: P2G of 250,007 particles in ~790 blocks 43.5 us
-    // instead of 36.7, of 328,509 in 343 blocks 47.9 instead of 43.2)
+    // (a block's parts side by side: P2G of 250,007 particles 44 us instead of 37, of
+    // 328,509 at 27 a cell 48 instead of 43.5, of 512,000 at 125 a cell 754 instead of 626;
+    // but of 884,736 at 27 a cell, in full blocks, 77 instead of 87)
     const int part = ONE ? wgl / nblocks : 0, b0 = wgl - part * nblocks;
     if (ONE ? part >= parts : b0 >= nblocks) return;
     int r0 = 0, r1 = 0; // ONE: the workgroup's part of its block's particles
@@ -2618,7 +2623,7 @@ struct RawG2P {
 // G2P's particle fields in two parts: what the gather needs (position and
 // material word) and what only the finish needs (F, m, V0, d, g, original
 // index, plastic state, J; FLIP: v).  The float form loads the second part
-// after the gather, so it is not live across it: 115 VGPRs, 4 wavefronts per
+// after the gather, so it is not live across it: 114 VGPRs, 4 wavefronts per
 // SIMD instead of 3 (G2P ~8 % faster); the double form, at 2
 // wavefronts either way, loads both up front.
 template <class T, class AccT>
@@ -2886,10 +2891,11 @@ __device__ __forceinline__ int blockRuns(const Dev<T, AccT>& D, int lo, int hi, 
 // they are dense, and dozens on a surface or in a sparse scene, where staging one
 // block after the other kept a workgroup for up to 135 us (mean 21): each block
 // is a chain of three dependent loads and a pass through the gather.  Eight
-// tiles are 27.6 KB (FP64 36.9 KB, FLIP the same with four): the four (two)
-// workgroups a CU holds by registers fit its LDS.  Measured with the gather and
+// tiles are 27.6 KB (FP64 36.9 KB, FLIP the same with four), 31.7 KB (42.8) with the
+// material table and the runs: the four (two) workgroups a CU holds by registers fit
+// its LDS.  Measured with the gather and
 // the finish compiled once each (a scene's table by wave-uniform pass and by
-// lane; 115 VGPRs, 18 KB of code less), event-timed, before -> after: 512 particles
+// lane; 114 VGPRs, 18 KB of code less), event-timed, before -> after: 512 particles
 // 30 -> 17 us, 130k FLIP 57 -> 27, 262k FP64 75 -> 47, 1M slab 87 -> 74, 4M
 // two-material column 437 -> 344, 10.4M batched scenes 912 -> 816.
 template <class T, bool FLIP> struct G2PTiles { static constexpr int value = FLIP ? 4 : 8; };
@@ -2898,8 +2904,12 @@ template <class T, bool FLIP> struct G2PTiles { static constexpr int value = FLI
 // XCD by XCD (an autotuner variant; results are the same).
 // FEW: the material table (at most G2P_FEW_MATS, as nearly every program's) is staged
 // in LDS: the finish reads a record many times, between its stores, and each read
-// from memory waits for the stores before it.
+// from memory waits for the stores before it.  Where the line lies matters little:
+// with 20 materials staged, G2P of 2M particles takes 135 us instead of 137, of
+// 262,144 24.8 instead of 25.2 and in FP64 49.9 instead of 48.7.
 constexpr int G2P_FEW_MATS = 16;
+// The FP64 FLIP form is held to two wavefronts per SIMD, at 20 VGPRs spilled: 30 us on
+// 130,001 particles, 145 on 1M, 52 on 262,144; without a spill at one wavefront 36, 166 and 67.
 
 template <class T, class AccT, bool FLIP, bool RR, bool FEW>
 __global__ __launch_bounds__(WG, sizeof(T) == 4 ? 4 : 2) void k_g2p(Dev<T, AccT> D)
@@ -3159,12 +3169,11 @@ __device__ __forceinline__ bool plasticMayProject(const MatDev<float>& mt, const
 }
 
 // The particles G2P deferred (queued by sorted position, the queues walked as
-// one list): the AnisoMPM damage
-// update on F_n with its full path (sigma^+, structural tensor) and the stress of
-// (F_{n+1}, g_{n+1}) with every branch of the models, and its force bound.  Runs
-// after k_g2p of the same substep, before the buffers swap.
-// P and Q: the live and output buffers of that G2P, qmat its output material words;
-// workgroup wg of nwg.
+// one list): the AnisoMPM damage update on F_n with its full path (sigma^+,
+// structural tensor) and the stress of (F_{n+1}, g_{n+1}) with every branch of the
+// models, and its force bound.  Runs after that k_g2p and before the next one's
+// P2G, on either side of the swap of the buffers: P and Q are that G2P's input and
+// output, qmat its output material words.  Workgroup wg of nwg.
 template <class T, class AccT>
 __device__ __forceinline__ void rareParticles(const Dev<T, AccT>& D, T* P, T* Q, const int* qmat, int wg, int nwg)
 {
