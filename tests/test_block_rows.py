@@ -4,7 +4,10 @@ import os
 import re
 import subprocess
 
+import numpy as np
 import pytest
+
+from ziran2020_amd import _abi as A, scenes
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "ziran2020_amd", "csrc")
@@ -43,3 +46,28 @@ def test_32_bit_accesses_start_at_a_row(table):
     text = open(os.path.join(CSRC, "zmpm_device.hpp")).read()
     assert not re.findall(r"\b(?:ldAt|stAt)\(D\.%s\b[^;]*;" % table, text)
     assert re.search(r"\bldAt\(blockRow<\w+>\(D\.%s, \w+\)" % table, text)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,per_axis", ((A.PREC_FP32, 131), (A.PREC_FP64, 163)))
+def test_lone_particles_in_blocks_past_the_wrap(gpu, monkeypatch, precision, per_axis):
+    """2.2M (4.3M) particles, each alone in eight blocks of its own: the last blocks are past the wrap, and
+    every particle falls as a free one does (the grid takes 130 to 160 GB)."""
+    n = per_axis ** 3
+    block_nodes = 64 if precision == A.PREC_FP32 else 32
+    assert 8 * n * block_nodes > 2 ** 30 + 2 ** 24
+    monkeypatch.setenv("ZMPM_BLOCK_CAPACITY", str(8 * n + 1000))
+    dx, dt, steps, g = 1 / 64, 1e-3, 3, np.array([0.0, -9.8, 0.0])
+    rng = np.random.default_rng(1)
+    site = np.stack(np.meshgrid(*[np.arange(per_axis) * 12 + 24] * 3, indexing="ij"), -1).reshape(-1, 3)
+    x = (site + 1.5 + rng.uniform(0.1, 0.9, (n, 3))) * dx
+    v = rng.uniform(-0.5, 0.5, (n, 3)).astype(np.float32).astype(float)
+    sim = A.Simulation(gpu, dx=dx, precision=precision, domain_nodes=2048, gravity=tuple(g))
+    sim.set_materials([A.make_material()])
+    sim.upload(x, v, np.zeros((n, 9)), scenes.identity_F(n), np.full(n, 1e-3), np.full(n, 1e-6), np.zeros(n, np.int32))
+    sim.run(steps, dt)
+    out = sim.download()
+    sim.close()
+    assert np.abs(out["v"] - (v + steps * dt * g)).max() < 1e-5
+    fall = dt * (steps * v + steps * (steps + 1) / 2 * dt * g)
+    assert np.abs(out["x"] - (x + fall)).max() < 1e-4 * dx
